@@ -4,7 +4,8 @@
 // IEEE-754 binary32 machine that provides a correctly rounded fma.
 //
 //   exp:    x = k ln2 + r, |r| <= ln2/2 (two-part ln2), Taylor to r^7,
-//           2^k applied in two exact scalings (subnormal results formed).
+//           2^k applied by one scaling, rounded once (subnormal results
+//           formed).
 //   sincos: q = rint(x * 2/pi), three-part pi/2 reduction, Taylor sin to
 //           r^9 and cos to r^10 on [-pi/4, pi/4], quadrant swap.
 //   cbrt:   bit-level seed, three Newton steps.
@@ -15,16 +16,15 @@ namespace oslmi {
 
 OSLMI_DEV float fexp(float x)
 {
-    if (!(x == x))
-        return x;
-    if (x > 88.72283935546875f)
-        return __uint_as_float(0x7f800000u);
-    if (x < -103.97208404541016f)
-        return 0.0f;
+    // No branch per special case: one wave evaluates several per point, and
+    // a branch costs it more than the whole range check. Above 88.7228 the
+    // scaling overflows to infinity by itself (k is held at 289, where the
+    // polynomial of what is left of x is at least 1), NaN passes through r;
+    // below -103.97 the result is selected.
     const float log2e  = 1.44269502162933349609375f;
     const float ln2_hi = 0.693145751953125f;
     const float ln2_lo = 1.428606765330187045e-06f;
-    float k            = rintf(x * log2e);
+    float k            = rintf(fminf(x, 200.0f) * log2e);
     float r            = __fmaf_rn(-k, ln2_hi, x);
     r                  = __fmaf_rn(-k, ln2_lo, r);
     float p            = 1.0f / 5040.0f;
@@ -35,12 +35,7 @@ OSLMI_DEV float fexp(float x)
     p                  = __fmaf_rn(p, r, 0.5f);
     p                  = __fmaf_rn(p, r, 1.0f);
     p                  = __fmaf_rn(p, r, 1.0f);
-    int ki             = (int)k;
-    int k1             = ki / 2;
-    int k2             = ki - k1;
-    float s1           = __uint_as_float((uint32_t)(k1 + 127) << 23);
-    float s2           = __uint_as_float((uint32_t)(k2 + 127) << 23);
-    return (p * s1) * s2;
+    return x < -103.97208404541016f ? 0.0f : ldexpf(p, (int)k);
 }
 
 OSLMI_DEV void fsincos(float x, float* s, float* c)
@@ -65,11 +60,13 @@ OSLMI_DEV void fsincos(float x, float* s, float* c)
     pc                      = __fmaf_rn(pc, r2, 1.0f / 24.0f);
     pc                      = __fmaf_rn(pc, r2, -0.5f);
     float cs                = __fmaf_rn(pc, r2, 1.0f);
-    int qi                  = ((int)q) & 3;
-    float sv = (qi == 0) ? sn : ((qi == 1) ? cs : ((qi == 2) ? -sn : -cs));
-    float cv = (qi == 0) ? cs : ((qi == 1) ? -sn : ((qi == 2) ? -cs : sn));
-    *s       = sv;
-    *c       = cv;
+    // quadrant q mod 4: odd ones swap sine and cosine, sine is negated in 2
+    // and 3, cosine in 1 and 2
+    const uint32_t qi = (uint32_t)(int)q;
+    const float sv    = (qi & 1u) ? cs : sn;
+    const float cv    = (qi & 1u) ? sn : cs;
+    *s = __uint_as_float(__float_as_uint(sv) ^ ((qi & 2u) << 30));
+    *c = __uint_as_float(__float_as_uint(cv) ^ (((qi + 1u) & 2u) << 30));
 }
 
 OSLMI_DEV float fcbrt(float x)
@@ -195,16 +192,10 @@ OSLMI_DEV float fierf(float x)
 }
 
 // 2^t: t = k + f, k = rint(t), 2^f by the Taylor series of e^(f ln2) to
-// degree 7, 2^k in two exact scalings.
+// degree 7, 2^k by one scaling. No branches, as in fexp.
 OSLMI_DEV float fexp2(float t)
 {
-    if (!(t == t))
-        return t;
-    if (t >= 128.0f)
-        return __uint_as_float(0x7f800000u);
-    if (t < -150.0f)
-        return 0.0f;
-    float k  = rintf(t);
+    float k  = rintf(fminf(t, 300.0f));
     float f  = t - k;
     float p  = 1.5252733804059840e-05f;
     p        = __fmaf_rn(p, f, 1.5403530393381608e-04f);
@@ -214,12 +205,7 @@ OSLMI_DEV float fexp2(float t)
     p        = __fmaf_rn(p, f, 2.4022650695910071e-01f);
     p        = __fmaf_rn(p, f, 6.9314718055994531e-01f);
     p        = __fmaf_rn(p, f, 1.0f);
-    int ki   = (int)k;
-    int k1   = ki / 2;
-    int k2   = ki - k1;
-    float s1 = __uint_as_float((uint32_t)(k1 + 127) << 23);
-    float s2 = __uint_as_float((uint32_t)(k2 + 127) << 23);
-    return (p * s1) * s2;
+    return t < -150.0f ? 0.0f : ldexpf(p, (int)k);
 }
 
 // x^y with fast_safe_pow's special cases (y == 0 -> 1, x == 0 -> 0,
@@ -227,19 +213,14 @@ OSLMI_DEV float fexp2(float t)
 // 2^(log2(x) y).
 OSLMI_DEV float fsafe_pow(float x, float y)
 {
-    if (y == 0.0f)
-        return 1.0f;
-    if (x == 0.0f)
-        return 0.0f;
-    if (y == 1.0f)
-        return x;
-    if (y == 2.0f) {
-        float x2 = x * x;
-        return x2 < 3.40282346638528859812e+38f ? x2 : 3.40282346638528859812e+38f;
-    }
-    if (x < 0.0f)
-        return 0.0f;
-    return fexp2(flog2(x) * y);
+    // the special cases are selected over the general value, last rule first
+    const float x2 = x * x;
+    float r        = fexp2(flog2(x) * y);
+    r              = x < 0.0f ? 0.0f : r;
+    r = y == 2.0f ? (x2 < 3.40282346638528859812e+38f ? x2 : 3.40282346638528859812e+38f) : r;
+    r = y == 1.0f ? x : r;
+    r = x == 0.0f ? 0.0f : r;
+    return y == 0.0f ? 1.0f : r;
 }
 
 // Dual2 exp and cos (dual.h:830-836, :1122-1127): f(a) with f'(a) * da.
