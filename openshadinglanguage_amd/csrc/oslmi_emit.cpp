@@ -68,6 +68,7 @@ struct Emitter {
     Group& g;
     std::string err;
     std::vector<std::vector<char>> deriv;  // [layer][sym]
+    std::vector<std::vector<char>> live;   // [layer][sym], see analyze_live
     std::ostringstream os;
     int label_counter = 0;
     std::string lprefix = "L";  // unique per group inside a batch kernel
@@ -437,6 +438,58 @@ struct Emitter {
         return k >= 0 && S(L, k).kind == kGlobal && S(L, k).type.base == kClosure ? k : -1;
     }
 
+    // Symbols whose value can reach a renderer output, a closure or a branch
+    // (flow-insensitive: a symbol counts as read by every op that may write
+    // a live one). The compiler drops dead arithmetic by itself, but not a
+    // Gabor noise, whose evaluation queues impulses in LDS; emit_noise leaves
+    // out one whose result is not live.
+    void analyze_live()
+    {
+        live.assign(g.layers.size(), {});
+        for (size_t L = 0; L < g.layers.size(); ++L)
+            live[L].assign(M((int)L).syms.size(), 0);
+        bool changed = true;
+        auto mark    = [&](int L, int s) {
+            if (!live[L][s]) {
+                live[L][s] = 1;
+                changed    = true;
+            }
+        };
+        for (size_t L = 0; L < g.layers.size(); ++L) {
+            const ShaderMaster& m = M((int)L);
+            for (size_t s = 0; s < m.syms.size(); ++s) {
+                bool root = m.syms[s].kind == kGlobal;
+                for (const std::string& o : g.output_names)
+                    root = root || o.substr(o.find_last_of('.') + 1) == m.syms[s].name;
+                if (root)
+                    mark((int)L, (int)s);
+            }
+            for (const OOp& op : m.ops)
+                if (op.jump[0] >= 0 && !op.args.empty())
+                    mark((int)L, op.args[0]);  // the condition of if / for / while / dowhile
+        }
+        while (changed) {
+            changed = false;
+            for (size_t L = 0; L < g.layers.size(); ++L)
+                for (const OOp& op : M((int)L).ops) {
+                    if (op.args.empty())
+                        continue;
+                    // results: the first argument, and the value arguments
+                    // of the two ops that return a status
+                    bool any = live[L][op.args[0]];
+                    if (op.name == "getattribute" || op.name == "getmatrix")
+                        for (int a : op.args)
+                            any = any || (S((int)L, a).kind != kConst && live[L][a]);
+                    if (any)
+                        for (int a : op.args)
+                            mark((int)L, a);
+                }
+            for (const Connection& c : g.conns)
+                if (live[c.dst_layer][c.dst_sym])
+                    mark(c.src_layer, c.src_sym);
+        }
+    }
+
     void analyze()
     {
         deriv.assign(g.layers.size(), {});
@@ -780,6 +833,8 @@ struct Emitter {
             line("}");
             return;
         }
+        if (nm == "gabor" && !live[L][r])
+            return;
         if (nm == "gabor") {
             GaborOptions go;
             for (size_t a = first + nnum; a + 1 < op.args.size(); a += 2) {
@@ -1417,6 +1472,7 @@ struct Emitter {
                 return false;
             }
         analyze();
+        analyze_live();
         g.uses_xforms = false;
         // outputs
         g.outputs.clear();

@@ -105,6 +105,7 @@ OSLMI_DEV Df ddot(V3 a, const Dv& b) { return comp(b, 0) * a.x + comp(b, 1) * a.
 
 struct GaborRng {
     uint32_t s;
+    OSLMI_DEV GaborRng() : s(1u) {}
     OSLMI_DEV GaborRng(V3 p, uint32_t seed)
     {
         s = inthash((uint32_t)ifloor(p.x), (uint32_t)ifloor(p.y), (uint32_t)ifloor(p.z), seed);
@@ -236,81 +237,366 @@ OSLMI_DEV Df gabor_impulse(const GaborUniform& U, const GaborPoint& gp, V3 omega
     return gabor_kernel3(omega, phi, U.a, xk);
 }
 
-// gabor_cell: impulses of one lattice cell, summed in generation order.
-// seed selects the generator stream (0 for the scalar noise, 0/1/2 for the
-// components of the vector noise); a periodic noise wraps the cell corner
-// before it seeds the generator (sfm_gabornoise.h:304-310).
-OSLMI_DEV Df gabor_cell(const GaborUniform& U, const GaborPoint& gp, V3 c_i, const Dv& x_c_i,
-                        uint32_t seed, bool periodic, V3 period)
+// ---- the impulse scan -----------------------------------------------------
+// An evaluation visits the cells around P, draws each cell's impulses and
+// adds up those within the kernel radius. The kernel of an impulse costs
+// 100 to 250 instructions, and one drawn impulse in six lies in the radius:
+// evaluated where it is found, the kernel runs for nearly every impulse of
+// every cell with a few of the 64 lanes active. So impulses that may lie in
+// the radius are queued per lane (generator state and cell, in LDS) and the
+// kernel runs over the queues when one is full and at the end. Terms keep
+// their order (cell after cell, summed per cell first), and the distance
+// test that decides is the kernel loop's, on the exact offset; the scan's
+// own test only has to keep every impulse that passes it.
+//
+// What is left is the scan, which has two forms:
+//  * per wave: the 64 lanes shade neighbouring points, whose cells fill a
+//    small box (at most 8 x 8 x 4 and 128 cells, every lane active). Each
+//    lane seeds the generator of one of the box's cells and draws its
+//    impulse count; then all lanes test every impulse of the box together.
+//    The generator runs once per wave, in the scalar unit, and nothing
+//    diverges;
+//  * per lane: each lane walks its own cells (points far apart, partly
+//    active waves).
+
+// Queue slots per lane: 10 slots of eight bytes for 256 work-items, 20 KB of
+// LDS: six workgroups a CU still fit, the six waves per SIMD that the
+// kernels are allocated for.
+constexpr int kGaborQueue = 10;
+struct GaborQueued {
+    uint32_t state, code;  // generator state before the impulse, its cell
+};
+
+// 3039177861^k modulo 2^32: k draws of the generator at once
+constexpr uint32_t gabor_rng_pow(int k)
 {
-    const float two_pi = 6.28318548202514648438f;
+    uint32_t r = 1u;
+    for (int i = 0; i < k; ++i)
+        r *= 3039177861u;
+    return r;
+}
+
+// The scan's distance test: squared distance of the impulse with generator
+// state s from the lane, both relative to the cell's centre and in units of
+// 2^-32 cells.
+OSLMI_DEV bool gabor_near(V3 in_cell, uint32_t s, float near2)
+{
+    const uint32_t half = 0x80000000u;
+    const V3 d = in_cell
+                 - V3((float)(int32_t)((s * gabor_rng_pow(3)) ^ half),
+                      (float)(int32_t)((s * gabor_rng_pow(2)) ^ half),
+                      (float)(int32_t)((s * gabor_rng_pow(1)) ^ half));
+    return __fmaf_rn(d.z, d.z, __fmaf_rn(d.y, d.y, d.x * d.x)) < near2;
+}
+
+// Poisson(lambda radius^3) by multiplying uniforms until the product is at
+// most g (fast_rng::poisson): n factors stay above g and the n + 1st does
+// not. The product never grows (no uniform exceeds 1), so n is the number
+// of partial products above g, counted here over four draws at a time:
+// the four states and products of a round do not wait for a branch each.
+OSLMI_DEV int gabor_poisson(GaborRng& rng, float g)
+{
+    const float k = 1.0f / 4294967296.0f;
+    int n   = 0;
+    float t = 1.0f;
+    for (;;) {
+        const uint32_t s1 = rng.s * gabor_rng_pow(1), s2 = rng.s * gabor_rng_pow(2);
+        const uint32_t s3 = rng.s * gabor_rng_pow(3), s4 = rng.s * gabor_rng_pow(4);
+        const float t1 = t * ((float)s1 * k), t2 = t1 * ((float)s2 * k);
+        const float t3 = t2 * ((float)s3 * k), t4 = t3 * ((float)s4 * k);
+        n += (t1 > g) + (t2 > g) + (t3 > g) + (t4 > g);
+        uint32_t s = s1;
+        s          = t1 > g ? s2 : s;
+        s          = t2 > g ? s3 : s;
+        s          = t3 > g ? s4 : s;
+        rng.s      = s;
+        if (!(t4 > g))
+            return n;
+        t = t4;
+    }
+}
+
+// Squared length of the smallest offset component that an impulse of the
+// cell at distance t = xc - c along one axis can have: the component is
+// radius * (t - u) with u in [0, 1], and rounding is monotone.
+OSLMI_DEV float gabor_axis_bound(const GaborUniform& U, float t)
+{
+    const float d = U.radius * (t < 0.0f ? t : (t > 1.0f ? t - 1.0f : 0.0f));
+    return d * d;
+}
+
+// The cells that can hold an impulse within the radius, as a bit each in
+// the order they are summed in (z outermost): a cell whose bounds already
+// give a squared length of radius2 or more contributes an exact zero. Of
+// the 27 cells 20.6 remain on average, 16.3 of a 1D or 2D noise (z = 0: the
+// cells above the plane touch the radius only).
+OSLMI_DEV uint32_t gabor_cell_mask(const GaborUniform& U, V3 xc)
+{
+    float sx[3], sy[3], sz[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        sx[a] = gabor_axis_bound(U, xc.x - (float)(a - 1));
+        sy[a] = gabor_axis_bound(U, xc.y - (float)(a - 1));
+        sz[a] = gabor_axis_bound(U, xc.z - (float)(a - 1));
+    }
+    uint32_t m = 0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                if (!((sx[i] + sy[j]) + sz[k] >= U.radius2))
+                    m |= 1u << (9 * k + 3 * j + i);
+    return m;
+}
+
+// Queued cells: box coordinates i, j < 8, k < 4 in one byte.
+OSLMI_DEV uint32_t gabor_cell_code(int i, int j, int k)
+{
+    return (uint32_t)(i | (j << 3) | (k << 6));
+}
+OSLMI_DEV V3 gabor_cell_of(uint32_t code)
+{
+    return V3((float)(code & 7u), (float)((code >> 3) & 7u), (float)(code >> 6));
+}
+
+// The generator of cell c_i, wrapped first by a periodic noise
+// (sfm_gabornoise.h:304-310).
+OSLMI_DEV GaborRng gabor_cell_rng(V3 c_i, uint32_t seed, bool periodic, V3 period)
+{
     if (periodic)
         c_i = V3(wrap_period(c_i.x, period.x), wrap_period(c_i.y, period.y),
                  wrap_period(c_i.z, period.z));
-    GaborRng rng(c_i, seed);
-    // Poisson(lambda*radius3) by multiplying uniforms (fast_rng::poisson)
-    int n = 0;
-    {
-        float t = rng();
-        while (t > U.poisson_g) {
-            ++n;
-            t *= rng();
-        }
-    }
-    Df sum = Df(0.0f);
-    for (int i = 0; i < n; ++i) {
-        float z_rng = rng(), y_rng = rng(), x_rng = rng();
-        V3 x_i_c(x_rng, y_rng, z_rng);
-        Dv xk = U.radius * Dv(x_c_i.v - x_i_c, x_c_i.dx, x_c_i.dy);
-        if (dot(xk.v, xk.v) < U.radius2) {
-            V3 omega;
-            if (U.anisotropic == 1) {
-                omega = V3(U.dir_x, U.dir_y, U.dir_z);
-            } else if (U.anisotropic == 0) {
-                float omega_t = two_pi * rng();
-                float u       = rng();
-                float cos_p   = -1.0f * (1.0f - u) + 1.0f * u;
-                float sin_p   = sqrtf(fmaxf(0.0f, 1.0f - cos_p * cos_p));
-                float st, ct;
-                fsincos(omega_t, &st, &ct);
-                omega = vnormalized(V3(ct * sin_p, st * sin_p, cos_p));
-            } else {
-                float omega_r = sqrtf(U.dir_x * U.dir_x + U.dir_y * U.dir_y + U.dir_z * U.dir_z);
-                float omega_t = two_pi * rng();
-                float st, ct;
-                fsincos(omega_t, &st, &ct);
-                omega = omega_r * V3(ct, st, 0.0f);
-            }
-            float phi = two_pi * rng();
-            sum       = sum + gabor_impulse(U, gp, omega, phi, xk);
-        } else {
-            if (U.anisotropic == 0) {
-                rng();
-                rng();
-            } else if (U.anisotropic != 1) {
-                rng();
-            }
-            rng();
-        }
-    }
-    return sum;
+    return GaborRng(c_i, seed);
 }
 
-// gabor_evaluate + gabor_grid: the 27 cells around P, scaled.
+// Smallest and largest value over the wave (all 64 lanes active), in every
+// lane's hands as a scalar.
+#if defined(__HIP_DEVICE_COMPILE__)
+template<bool MAX> OSLMI_DEV int wave_extreme(int v)
+{
+#define OSLMI_EXTREME_STEP(ctrl)                                                     \
+    {                                                                                \
+        const int o = __builtin_amdgcn_update_dpp(v, v, ctrl, 0xf, 0xf, false);      \
+        v           = (MAX ? o > v : o < v) ? o : v;                                 \
+    }
+    OSLMI_EXTREME_STEP(0x111)  // row_shr:1, 2, 4, 8
+    OSLMI_EXTREME_STEP(0x112)
+    OSLMI_EXTREME_STEP(0x114)
+    OSLMI_EXTREME_STEP(0x118)
+    OSLMI_EXTREME_STEP(0x142)  // row_bcast:15, 31
+    OSLMI_EXTREME_STEP(0x143)
+#undef OSLMI_EXTREME_STEP
+    return __builtin_amdgcn_readlane(v, 63);
+}
+#endif
+
+// The wave's box of cells: origin (ox, oy, oz), size (dx, dy, dz). False
+// where the per-wave scan does not apply. An axis reaches one cell beyond
+// the lanes' own cells on either side, above only where a lane needs it.
+struct GaborBox {
+    int ox, oy, oz, dx, dy, dz;
+};
+OSLMI_DEV bool gabor_wave_box(const GaborUniform& U, V3 fl, V3 xc, GaborBox& b)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (__ballot(1) != ~0ull)
+        return false;
+    // cells a binary32 coordinate and an int hold alike (false for NaN)
+    const float lim = 1048576.0f;
+    if (wave_any(!(fabsf(fl.x) < lim && fabsf(fl.y) < lim && fabsf(fl.z) < lim)))
+        return false;
+    const int x = (int)fl.x, y = (int)fl.y, z = (int)fl.z;
+    b.ox = wave_extreme<false>(x) - 1;
+    b.dx = wave_extreme<true>(x) + 2 - b.ox;
+    if (b.dx > 8)
+        return false;
+    b.oy = wave_extreme<false>(y) - 1;
+    b.dy = wave_extreme<true>(y) + 2 - b.oy;
+    b.oz = wave_extreme<false>(z) - 1;
+    b.dz = wave_extreme<true>(gabor_axis_bound(U, xc.z - 1.0f) >= U.radius2 ? z : z + 1) + 1 - b.oz;
+    return b.dy <= 8 && b.dz <= 4 && b.dx * b.dy * b.dz <= 128;
+#else
+    return false;
+#endif
+}
+
+// gabor_evaluate + gabor_grid: the cells around P, scaled. seed selects the
+// generator stream (0 for the scalar noise, 0/1/2 for the components of the
+// vector noise).
 OSLMI_DEV Df gabor_grid(const GaborUniform& U, const GaborPoint& gp, const Dv& P, uint32_t seed,
                         bool periodic, V3 period)
 {
+    const float two_pi = 6.28318548202514648438f;
+    const float two32  = 4294967296.0f;
+    // the scan's squared distance limit, in units of 2^32 cells: 1 + 2^-10
+    // lets every impulse through whose exact offset is inside (the scan's
+    // rounding errors are below 2^-18)
+    const float near2 = 1.0009765625f * two32 * two32;
+    __shared__ GaborQueued queue[kGaborQueue][256];
+    const int tid = (int)threadIdx.x;
+    // draws per impulse: position, direction (isotropic 2, hybrid 1), phase
+    const uint32_t step = U.anisotropic == 1   ? gabor_rng_pow(4)
+                          : U.anisotropic == 0 ? gabor_rng_pow(6)
+                                               : gabor_rng_pow(5);
     Dv xg = P * U.radius_inv;
     V3 fl(floorf(xg.v.x), floorf(xg.v.y), floorf(xg.v.z));
     Dv xc(xg.v - fl, xg.dx, xg.dy);
-    Df sum = Df(0.0f);
-    for (int k = -1; k <= 1; ++k)
-        for (int j = -1; j <= 1; ++j)
-            for (int i = -1; i <= 1; ++i) {
-                V3 c((float)i, (float)j, (float)k);
-                sum = sum + gabor_cell(U, gp, fl + c, Dv(xc.v - c, xc.dx, xc.dy), seed, periodic,
-                                       period);
+    GaborBox box = { 0, 0, 0, 0, 0, 0 };
+    const bool by_wave = gabor_wave_box(U, fl, xc.v, box);
+    // the queued cells' origin relative to this lane's cell, and the lane's
+    // position from that cell's centre in units of 2^-32 cells
+    V3 org(-1.0f, -1.0f, -1.0f);
+    uint32_t cells = 0;
+    if (by_wave) {
+        org = V3((float)box.ox, (float)box.oy, (float)box.oz) - fl;
+    } else {
+        cells = gabor_cell_mask(U, xc.v);
+    }
+    const V3 at = two32 * (xc.v - org) - V3(0.5f * two32);
+    // the same from the centre of the cell being scanned
+    V3 in_cell = at;
+    // per lane: its cell's code, generator state and impulses left
+    uint32_t code = 0, state = 0;
+    int left = 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+    // per wave: the same of the wave's cell (wi, wj, wk), the cell-th of
+    // ncells; and the cells cell / 64 * 64 + lane, one per lane
+    const int ncells = box.dx * box.dy * box.dz;
+    int cell = 0, wi = 0, wj = 0, wk = 0, wleft = 0, lane_count = 0;
+    uint32_t wcode = 0, wstate = 0, lane_state = 0;
+    V3 wpos = at;
+#endif
+    int queued = 0, sum_code = -1;
+    Df sum = Df(0.0f), cell_sum = Df(0.0f);
+    for (;;) {
+        bool last;
+#if defined(__HIP_DEVICE_COMPILE__)
+        if (by_wave) {
+            if (wleft <= 0 && cell < ncells) {
+                if ((cell & 63) == 0) {
+                    const int mine = cell + (int)__lane_id();
+                    const int q = mine / box.dx, k = q / box.dy;
+                    GaborRng rng = gabor_cell_rng(
+                        V3((float)(box.ox + mine - q * box.dx), (float)(box.oy + q - k * box.dy),
+                           (float)(box.oz + k)),
+                        seed, periodic, period);
+                    lane_count = mine < ncells ? gabor_poisson(rng, U.poisson_g) : 0;
+                    lane_state = rng.s;
+                }
+                // left out when no lane is within a cell's width of the cell
+                if (wave_any(fmaxf(fmaxf(fabsf(wpos.x), fabsf(wpos.y)), fabsf(wpos.z))
+                             < 1.50001f * two32)) {
+                    wleft   = __builtin_amdgcn_readlane(lane_count, cell & 63);
+                    wstate  = (uint32_t)__builtin_amdgcn_readlane((int)lane_state, cell & 63);
+                    in_cell = wpos;
+                    wcode   = gabor_cell_code(wi, wj, wk);
+                }
+                // on to the next cell, x innermost
+                ++cell;
+                wpos.x -= two32;
+                if (++wi == box.dx) {
+                    wi     = 0;
+                    wpos.x = at.x;
+                    wpos.y -= two32;
+                    if (++wj == box.dy) {
+                        wj     = 0;
+                        wpos.y = at.y;
+                        wpos.z -= two32;
+                        ++wk;
+                    }
+                }
             }
+            // two impulses a round; a slot is written whether or not the
+            // impulse is kept, so nothing branches
+            bool full = false;
+            while (wleft > 0 && !full) {
+                const uint32_t next = wstate * step;
+                queue[queued][tid]  = GaborQueued { wstate, wcode };
+                queued += gabor_near(in_cell, wstate, near2);
+                queue[queued][tid] = GaborQueued { next, wcode };
+                queued += wleft > 1 && gabor_near(in_cell, next, near2);
+                wstate = (uint32_t)__builtin_amdgcn_readfirstlane((int)(next * step));
+                wleft -= 2;
+                full = wave_any(queued > kGaborQueue - 2);
+            }
+            last = wleft <= 0 && cell >= ncells;
+            if (!last && !full)
+                continue;
+        } else
+#endif
+        {
+            if (!wave_any(left > 0) && cells) {
+                const int bit = __builtin_ctz(cells);
+                cells &= cells - 1;
+                const int q = (bit * 171) >> 9;  // bit / 3
+                const int k = (q * 171) >> 9;
+                code        = gabor_cell_code(bit - 3 * q, q - 3 * k, k);
+                const V3 c  = gabor_cell_of(code);
+                in_cell     = at - two32 * c;
+                GaborRng rng = gabor_cell_rng(fl + (org + c), seed, periodic, period);
+                left         = gabor_poisson(rng, U.poisson_g);
+                state        = rng.s;
+            }
+            while (wave_any(left > 0) && !wave_any(queued > kGaborQueue - 2)) {
+                const uint32_t next = state * step;
+                queue[queued][tid]  = GaborQueued { state, code };
+                queued += left > 0 && gabor_near(in_cell, state, near2);
+                queue[queued][tid] = GaborQueued { next, code };
+                queued += left > 1 && gabor_near(in_cell, next, near2);
+                state = next * step;
+                left -= 2;
+            }
+            last = !wave_any(cells != 0 || left > 0);
+            if (!last && !wave_any(queued > kGaborQueue - 2))
+                continue;
+        }
+#pragma clang loop unroll(disable)
+        for (int e = 0; wave_any(e < queued); ++e) {
+            if (e < queued) {
+                GaborRng rng;
+                const GaborQueued it = queue[e][tid];
+                rng.s                = it.state;
+                const uint32_t qc    = it.code;
+                const V3 c        = org + gabor_cell_of(qc);
+                const float z_rng = rng(), y_rng = rng(), x_rng = rng();
+                const Dv xk = U.radius * Dv((xc.v - c) - V3(x_rng, y_rng, z_rng), xc.dx, xc.dy);
+                if (dot(xk.v, xk.v) < U.radius2) {
+                    if ((int)qc != sum_code) {
+                        sum      = sum + cell_sum;
+                        cell_sum = Df(0.0f);
+                        sum_code = (int)qc;
+                    }
+                    V3 omega;
+                    if (U.anisotropic == 1) {
+                        omega = V3(U.dir_x, U.dir_y, U.dir_z);
+                    } else if (U.anisotropic == 0) {
+                        float omega_t = two_pi * rng();
+                        float u       = rng();
+                        float cos_p   = -1.0f * (1.0f - u) + 1.0f * u;
+                        float sin_p   = sqrtf(fmaxf(0.0f, 1.0f - cos_p * cos_p));
+                        float st, ct;
+                        fsincos(omega_t, &st, &ct);
+                        omega = vnormalized(V3(ct * sin_p, st * sin_p, cos_p));
+                    } else {
+                        float omega_r
+                            = sqrtf(U.dir_x * U.dir_x + U.dir_y * U.dir_y + U.dir_z * U.dir_z);
+                        float omega_t = two_pi * rng();
+                        float st, ct;
+                        fsincos(omega_t, &st, &ct);
+                        omega = omega_r * V3(ct, st, 0.0f);
+                    }
+                    const float phi = two_pi * rng();
+                    cell_sum        = cell_sum + gabor_impulse(U, gp, omega, phi, xk);
+                }
+            }
+        }
+        queued = 0;
+        if (last)
+            break;
+    }
+    sum = sum + cell_sum;
     return (sum * U.sqrt_lambda_inv) * U.scale;
 }
 

@@ -30,6 +30,17 @@ typedef __hip_internal::uint64_t uint64_t;
 
 namespace oslmi {
 
+// Whether the predicate holds in any active lane of the wave (one lane
+// where the kernels are built for the host).
+OSLMI_DEV bool wave_any(bool p)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __any(p) != 0;
+#else
+    return p;
+#endif
+}
+
 struct V3 {
     float x, y, z;
     OSLMI_HD V3() : x(0.f), y(0.f), z(0.f) {}
