@@ -158,7 +158,7 @@ void bake_tables(float* out)
         sp.eta = dfresnel_eta(LERP(SQR(findex), kIOR_MIN, kIOR_MAX), false);
         for (int c = 0; c < kNc; c++) {
             const float cth = get_cosine(kLutReflFront, c);
-            sp.E_ms         = emiss_eval(out, kLutMiniGGX, rough, 0.0f, cth);
+            sp.msf          = ms_factor(emiss_eval(out, kLutMiniGGX, rough, 0.0f, cth));
             auto w          = [&](V3 wo, V3 rnd) {
                 if (wo.z <= 0)
                     return 0.0f;
@@ -279,6 +279,7 @@ struct Layered {
     V3 s_tint;
     float s_a, s_Emiss;
     MicroLobe coat, base;
+    WoTerms coat_t, base_t;
     int n;  // lobes present: sheen, then coat, then base
     V3 w[3];
     float pdf[3];
@@ -291,17 +292,22 @@ OSLMI_DEV Sample sheen_eval(const Layered& L, V3 wo, V3 wi)
         return zero_sample();
     return sheen_mf_eval(L.s_a, L.s_tint, wo, wi);
 }
-// DielectricLobe / SchlickLobe ::eval_impl, reflection only
-OSLMI_DEV Sample micro_eval(const MicroLobe& M, V3 wo, V3 wi)
+// DielectricLobe / SchlickLobe ::eval_impl, reflection only, of the
+// geometry r
+OSLMI_DEV Sample micro_eval(const MicroLobe& M, const Refl& r)
 {
     if (!M.dorefl)
         return zero_sample();
-    Sample s = eval_turquin(M.sp, wo, wi);
+    Sample s = turquin_weight(M.sp, r);
     s.weight = s.weight * (s.wi.z > 0 ? M.tint : V3(0.0f));
     return s;
 }
 
-OSLMI_DEV void micro_setup(MicroLobe* M, float roughness_xy, float cosNO, const float* T)
+// The two microfacet lobes' roughness state. SAME: coat and base have one
+// roughness (the material's base_roughness is negative), so one distribution
+// and one set of wo terms serve both; a lookup or length less per point, and
+// one geometry less wherever both are evaluated at one direction.
+OSLMI_DEV float micro_rough(MicroLobe* M, float roughness_xy)
 {
     const float rx    = CLAMP(roughness_xy, kEPSILON, 2.0f);
     const float ry    = rx;
@@ -311,12 +317,15 @@ OSLMI_DEV void micro_setup(MicroLobe* M, float roughness_xy, float cosNO, const 
     const float aniso = (1 - b) / (1 + b);
     const float rough = regularize_roughness(sqrtf(ax / (1 + aniso)));
     M->sp.d           = ggx_make(rough, aniso, rx < ry);
-    M->sp.E_ms        = emiss_eval(T, kLutMiniGGX, rough, 0.0f, cosNO);
-    M->E_ms           = M->dorefl ? emiss_eval(T, kLutReflFront, rough,
-                                               dfresnel_table_index(M->sp.eta), cosNO)
-                                  : 0.0f;
+    return rough;
+}
+OSLMI_DEV void micro_energy(MicroLobe* M, float rough, float cosNO, const float* T)
+{
+    M->E_ms = M->dorefl ? emiss_eval(T, kLutReflFront, rough, dfresnel_table_index(M->sp.eta), cosNO)
+                        : 0.0f;
 }
 
+template<bool SAME>
 OSLMI_DEV void layered_build(Layered* L, const Material& mat, V3 N, V3 wo, float coat_ior,
                              float coat_rough, float sheen_rough, V3 F0, V3 F90, const float* T)
 {
@@ -339,7 +348,10 @@ OSLMI_DEV void layered_build(Layered* L, const Material& mat, V3 N, V3 wo, float
     L->coat.sp.eta  = dfresnel_eta(CLAMP(coat_ior, kIOR_MIN, kIOR_MAX) / 1.0f, false);
     L->coat.sp.F0 = L->coat.sp.F90 = V3(0.0f);
     L->coat.sp.exponent = L->coat.sp.tir_cos = 0.0f;
-    micro_setup(&L->coat, coat_rough, cosNO, T);
+    const float c_rough = micro_rough(&L->coat, coat_rough);
+    L->coat.sp.msf      = ms_factor(emiss_eval(T, kLutMiniGGX, c_rough, 0.0f, cosNO));
+    L->coat_t           = ggx_wo_terms(L->coat.sp.d, L->wo_m);
+    micro_energy(&L->coat, c_rough, cosNO, T);
     // generalized_schlick_bsdf base
     const float avg_F0 = CLAMP((F0.x + F0.y + F0.z) * (1.0f / 3), 0.0f, 0.99f);
     const float sqF0   = sqrtf(avg_F0);
@@ -353,7 +365,17 @@ OSLMI_DEV void layered_build(Layered* L, const Material& mat, V3 N, V3 wo, float
                         smax(0.0f, smin(1.0f, F90.z)));
     L->base.sp.exponent = mat.base_exponent;
     L->base.sp.tir_cos  = L->base.sp.eta >= 1 ? 0 : sqrtf(1 - SQR(L->base.sp.eta));
-    micro_setup(&L->base, mat.base_roughness < 0 ? coat_rough : mat.base_roughness, cosNO, T);
+    float b_rough       = c_rough;
+    if (SAME) {
+        L->base.sp.d   = L->coat.sp.d;
+        L->base.sp.msf = L->coat.sp.msf;
+        L->base_t      = L->coat_t;
+    } else {
+        b_rough        = micro_rough(&L->base, mat.base_roughness);
+        L->base.sp.msf = ms_factor(emiss_eval(T, kLutMiniGGX, b_rough, 0.0f, cosNO));
+        L->base_t      = ggx_wo_terms(L->base.sp.d, L->wo_m);
+    }
+    micro_energy(&L->base, b_rough, cosNO, T);
     // layer weights: top opacity = 1 - filter_o, clamped (closure weights 1)
     const V3 one(1.0f);
     auto oclamp = [](float a) {
@@ -416,27 +438,35 @@ OSLMI_DEV void mis_update(V3* w, float* pdf, V3 ow, float opdf, float b)
         *pdf += opdf;
     }
 }
-
-// lobe i evaluated at the local directions of its frame
-OSLMI_DEV Sample lobe_eval_local(const Layered& L, int i, V3 wi_local)
+// mis_update of a zero weight and pdf (the sheen, evaluated first): its two
+// quotients are 0 and 1
+OSLMI_DEV void mis_first(V3* w, float* pdf, V3 ow, float opdf, float b)
 {
-    if (i == 0)
-        return sheen_eval(L, L.wo_s, wi_local);
-    return micro_eval(i == 1 ? L.coat : L.base, L.wo_m, wi_local);
+    if (b > kFLT_MIN) {
+        opdf *= b;
+        ow              = ow * (1 / b);
+        const float mis = 0.0f < opdf ? 1.0f : 0.5f;
+        *w              = V3(0.0f) + ow * mis;
+        *pdf            = opdf;
+    }
 }
 
 // CompositeBSDF::eval at world direction wi: weight rgb, pdf
-OSLMI_DEV void layered_eval(const Layered& L, V3 wi, V3* weight, float* pdf)
+template<bool SAME> OSLMI_DEV void layered_eval(const Layered& L, V3 wi, V3* weight, float* pdf)
 {
     V3 sw(0.0f);
-    float sp        = 0.0f;
-    const V3 wi_s   = L.fs.local(wi);
-    const V3 wi_m   = L.fm.local(wi);
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        if (i < L.n) {
-            Sample b = lobe_eval_local(L, i, i == 0 ? wi_s : wi_m);
-            mis_update(&sw, &sp, b.weight * L.w[i], b.pdf, L.pdf[i]);
+    float sp      = 0.0f;
+    const V3 wi_s = L.fs.local(wi);
+    const V3 wi_m = L.fm.local(wi);
+    Sample b      = sheen_eval(L, L.wo_s, wi_s);
+    mis_first(&sw, &sp, b.weight * L.w[0], b.pdf, L.pdf[0]);
+    if (L.n > 1) {
+        const Refl g = turquin_geometry(L.coat.sp.d, L.coat_t, L.wo_m, wi_m);
+        b            = micro_eval(L.coat, g);
+        mis_update(&sw, &sp, b.weight * L.w[1], b.pdf, L.pdf[1]);
+        if (L.n > 2) {
+            b = micro_eval(L.base, SAME ? g : turquin_geometry(L.base.sp.d, L.base_t, L.wo_m, wi_m));
+            mis_update(&sw, &sp, b.weight * L.w[2], b.pdf, L.pdf[2]);
         }
     }
     *weight = sw;
@@ -484,13 +514,14 @@ OSLMI_DEV void layered_sample(const Layered& L, float rx, float ry, V3* wi_out, 
     const Frame& f = pick == 0 ? L.fs : L.fm;
     const V3 wi    = f.world(wl);
     Sample b[3];
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-        if (j < L.n) {
-            V3 d = j == pick ? wl : (j == 0 ? L.fs.local(wi) : L.fm.local(wi));
-            b[j] = lobe_eval_local(L, j, d);
-        }
-    }
+    b[0] = sheen_eval(L, L.wo_s, pick == 0 ? wl : L.fs.local(wi));
+    const V3 wi_m = L.fm.local(wi);
+    if (L.n > 1)
+        b[1] = micro_eval(L.coat, turquin_geometry(L.coat.sp.d, L.coat_t, L.wo_m,
+                                                   pick == 1 ? wl : wi_m));
+    if (L.n > 2)
+        b[2] = micro_eval(L.base, turquin_geometry(L.base.sp.d, L.base_t, L.wo_m,
+                                                   pick == 2 ? wl : wi_m));
     V3 sw    = V3(0.0f);
     float sp = 0.0f;
 #pragma unroll
@@ -513,6 +544,7 @@ OSLMI_DEV void layered_sample(const Layered& L, float rx, float ry, V3* wi_out, 
 
 // ---- kernels ---------------------------------------------------------------
 // Tables staged in LDS: 8448 floats (33 KB) per workgroup.
+template<bool SAME>
 __global__ __launch_bounds__(kLayeredBlock) void k_layered(Material mat, const float* __restrict__ lut,
                                                  const float* __restrict__ Np,
                                                  const float* __restrict__ Vp,
@@ -531,13 +563,13 @@ __global__ __launch_bounds__(kLayeredBlock) void k_layered(Material mat, const f
         const V3 N(Np[i], Np[n + i], Np[2 * n + i]);
         const V3 wo(Vp[i], Vp[n + i], Vp[2 * n + i]);
         Layered L;
-        layered_build(&L, mat, N, wo, prm[i], prm[n + i], prm[2 * n + i],
+        layered_build<SAME>(&L, mat, N, wo, prm[i], prm[n + i], prm[2 * n + i],
                       V3(prm[3 * n + i], prm[4 * n + i], prm[5 * n + i]),
                       V3(prm[6 * n + i], prm[7 * n + i], prm[8 * n + i]), T);
         if (eval) {
             V3 w;
             float p;
-            layered_eval(L, V3(Lp[i], Lp[n + i], Lp[2 * n + i]), &w, &p);
+            layered_eval<SAME>(L, V3(Lp[i], Lp[n + i], Lp[2 * n + i]), &w, &p);
             eval[i]         = w.x;
             eval[n + i]     = w.y;
             eval[2 * n + i] = w.z;
@@ -565,47 +597,41 @@ __global__ __launch_bounds__(kLayeredBlock) void k_layered(Material mat, const f
 // Exact evaluation of surrogate queries in the local frame (N = +z,
 // wo = (x, 0, z)): q 14 planes = wi xyz, wo x z, coat ior, coat roughness,
 // sheen roughness, F0 rgb, F90 rgb; out 4 planes = weight rgb, pdf.
+template<bool SAME>
 OSLMI_DEV void eval_query(const Material& mat, const float* T, const float* __restrict__ q,
                           int64_t n, int64_t i, float* __restrict__ out)
 {
-    const float lz = q[2 * n + i], vz = q[4 * n + i];
-    if (vz > 0.0f && lz <= 0.0f) {
-        // N = +z is the visible normal and every lobe is reflection-only:
-        // the composite's weight and pdf are exactly zero
-        out[i] = out[n + i] = out[2 * n + i] = out[3 * n + i] = 0.0f;
-        return;
-    }
     const float* p = q + 5 * n;
     Layered L;
-    layered_build(&L, mat, V3(0.0f, 0.0f, 1.0f), V3(q[3 * n + i], 0.0f, vz), p[i], p[n + i],
-                  p[2 * n + i], V3(p[3 * n + i], p[4 * n + i], p[5 * n + i]),
-                  V3(p[6 * n + i], p[7 * n + i], p[8 * n + i]), T);
+    layered_build<SAME>(&L, mat, V3(0.0f, 0.0f, 1.0f), V3(q[3 * n + i], 0.0f, q[4 * n + i]), p[i],
+                        p[n + i], p[2 * n + i], V3(p[3 * n + i], p[4 * n + i], p[5 * n + i]),
+                        V3(p[6 * n + i], p[7 * n + i], p[8 * n + i]), T);
     V3 w;
     float pdf;
-    layered_eval(L, V3(q[i], q[n + i], lz), &w, &pdf);
+    layered_eval<SAME>(L, V3(q[i], q[n + i], q[2 * n + i]), &w, &pdf);
     out[i]         = w.x;
     out[n + i]     = w.y;
     out[2 * n + i] = w.z;
     out[3 * n + i] = pdf;
 }
 
-__global__ __launch_bounds__(kLocalBlock) void k_layered_local(Material mat,
-                                                       const float* __restrict__ lut,
-                                                       const float* __restrict__ q,
-                                                       float* __restrict__ out, int64_t n)
+// Query i of a list or range. V above and L below the surface: N = +z is
+// the visible normal and every lobe is reflection-only, so weight and pdf
+// are exactly zero.
+OSLMI_DEV bool query_is_zero(const float* __restrict__ q, int64_t n, int64_t i)
 {
-    __shared__ float T[kLutFloats];
-    for (int k = threadIdx.x; k < kLutFloats; k += blockDim.x)
-        T[k] = lut[k];
-    __syncthreads();
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-        eval_query(mat, T, q, n, i, out);
+    return q[4 * n + i] > 0.0f && q[2 * n + i] <= 0.0f;
 }
 
-// The same over the query indices idx[0 .. *count) (count written on the
-// device by an earlier kernel on the stream; every index < n).
-__global__ __launch_bounds__(kLocalBlock) void k_layered_local_indexed(Material mat,
+// n queries, or with idx the queries idx[0 .. *count) (count written on the
+// device by an earlier kernel on the stream; entries outside [0, n) are
+// passed over). Each wave reads 64 queries at a time, answers those that are
+// exactly zero (half of the directions of a uniform sphere) and keeps the
+// others in a ring in LDS; the closure runs on 64 of them at once, so no
+// lane of it idles on a zero.
+constexpr int kQueryRing = 128;
+template<bool SAME>
+__global__ __launch_bounds__(kLocalBlock) void k_layered_local(Material mat,
                                                                const float* __restrict__ lut,
                                                                const float* __restrict__ q,
                                                                int64_t n,
@@ -614,17 +640,43 @@ __global__ __launch_bounds__(kLocalBlock) void k_layered_local_indexed(Material 
                                                                float* __restrict__ out)
 {
     __shared__ float T[kLutFloats];
-    const int64_t cnt = *count;
+    __shared__ int64_t s_ring[kLocalBlock / 64][kQueryRing];
+    const int64_t cnt = idx ? (int64_t)*count : n;
     if ((int64_t)blockIdx.x * blockDim.x >= cnt)
         return;
     for (int k = threadIdx.x; k < kLutFloats; k += blockDim.x)
         T[k] = lut[k];
     __syncthreads();
+    const int lane = threadIdx.x & 63;
+    int64_t* ring  = s_ring[threadIdx.x >> 6];
+    int head = 0, pending = 0;  // the same in every lane of the wave
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += stride) {
-        const int64_t qi = idx[i];
-        if (qi >= 0 && qi < n)
-            eval_query(mat, T, q, n, qi, out);
+    int64_t first        = (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63);
+    while (first < cnt || pending > 0) {
+        if (first < cnt) {
+            const int64_t k = first + lane;
+            int64_t i       = k < cnt ? (idx ? (int64_t)idx[k] : k) : -1;
+            if (i >= n)
+                i = -1;
+            const bool zero = i >= 0 && query_is_zero(q, n, i);
+            if (zero)
+                out[i] = out[n + i] = out[2 * n + i] = out[3 * n + i] = 0.0f;
+            const bool keep            = i >= 0 && !zero;
+            const unsigned long long m = __ballot(keep);
+            if (keep)
+                ring[(head + pending + __popcll(m & ((1ull << lane) - 1ull))) % kQueryRing] = i;
+            pending += __popcll(m);
+            first += stride;
+            __builtin_amdgcn_wave_barrier();
+            if (pending < 64 && first < cnt)
+                continue;
+        }
+        if (lane < pending)
+            eval_query<SAME>(mat, T, q, n, ring[(head + lane) % kQueryRing], out);
+        const int done = pending < 64 ? pending : 64;
+        head           = (head + done) % kQueryRing;
+        pending -= done;
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -657,6 +709,16 @@ static int material_of(const oslmi_layered_material* m, mtx::Material* out, cons
     return OSLMI_OK;
 }
 
+static int launch_local(const mtx::Material& mat, const float* lut, const float* d_query, int64_t n,
+                        const int* d_index, const int* d_count, float* d_out, hipStream_t stream,
+                        const char* who)
+{
+    hipLaunchKernelGGL(mat.base_roughness < 0 ? mtx::k_layered_local<true> : mtx::k_layered_local<false>,
+                       dim3(layered_grid(n, kLocalBlock)), dim3(kLocalBlock), 0, stream, mat, lut,
+                       d_query, n, d_index, d_count, d_out);
+    return check_launch(who);
+}
+
 // Exact evaluation of the queries listed in d_index[0 .. *d_count) (the
 // surrogate's fallback list); the grid covers up to n listed queries.
 int layered_eval_local_indexed(const oslmi_layered_material* m, int64_t n, const float* d_query,
@@ -669,9 +731,7 @@ int layered_eval_local_indexed(const oslmi_layered_material* m, int64_t n, const
     const float* lut = nullptr;
     if (int rc = mtx::device_tables(&lut))
         return rc;
-    hipLaunchKernelGGL(mtx::k_layered_local_indexed, dim3(layered_grid(n, kLocalBlock)), dim3(kLocalBlock),
-                       0, stream, mat, lut, d_query, n, d_index, d_count, d_out);
-    return check_launch("surrogate fallback");
+    return launch_local(mat, lut, d_query, n, d_index, d_count, d_out, stream, "surrogate fallback");
 }
 
 }  // namespace oslmi
@@ -695,7 +755,8 @@ extern "C" int oslmi_layered_closure(const oslmi_layered_material* m, int64_t n,
     const float* lut = nullptr;
     if (int rc = mtx::device_tables(&lut))
         return rc;
-    hipLaunchKernelGGL(mtx::k_layered, dim3(layered_grid(n, kLayeredBlock)), dim3(kLayeredBlock), 0,
+    hipLaunchKernelGGL(mat.base_roughness < 0 ? mtx::k_layered<true> : mtx::k_layered<false>,
+                       dim3(layered_grid(n, kLayeredBlock)), dim3(kLayeredBlock), 0,
                        (hipStream_t)stream, mat, lut, d_N, d_V, d_L, d_params, d_rnd, d_eval, d_samples, n);
     return check_launch("oslmi_layered_closure");
 }
@@ -715,9 +776,8 @@ extern "C" int oslmi_layered_eval_local(const oslmi_layered_material* m, int64_t
     const float* lut = nullptr;
     if (int rc = mtx::device_tables(&lut))
         return rc;
-    hipLaunchKernelGGL(mtx::k_layered_local, dim3(layered_grid(n, kLocalBlock)), dim3(kLocalBlock), 0,
-                       (hipStream_t)stream, mat, lut, d_query, d_out, n);
-    return check_launch("oslmi_layered_eval_local");
+    return launch_local(mat, lut, d_query, n, nullptr, nullptr, d_out, (hipStream_t)stream,
+                        "oslmi_layered_eval_local");
 }
 
 extern "C" int oslmi_bsdl_tables(float* out, int64_t count)

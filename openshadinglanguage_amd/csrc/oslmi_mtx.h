@@ -227,11 +227,6 @@ OSLMI_HD float ggx_D(const GGX& d, V3 Hr)
     const float sinThetaM2 = cosPhi2st2 + sinPhi2st2;
     return 1.0f / (kPI * d.ax * d.ay * SQR(cosThetaM2 + sinThetaM2));
 }
-OSLMI_HD float ggx_G1(const GGX& d, V3 w)
-{
-    w = V3(w.x * d.ax, w.y * d.ay, w.z);
-    return 2.0f * w.z / (w.z + vlength(w));
-}
 OSLMI_HD float ggx_G2_G1(const GGX& d, V3 wi, V3 wo)
 {
     wi             = V3(wi.x * d.ax, wi.y * d.ay, wi.z);
@@ -251,6 +246,20 @@ OSLMI_HD float ggx_D_refl_D(const GGX& d, V3 wo)
     const float s2   = SQR(s);
     const float k    = (1 - a2) * s2 / (s2 + a2 * SQR(wo.z));
     return 2 * wo.z / (k * wo.z + t);
+}
+// What a reflection eval needs of wo alone: the length of the stretched wo,
+// G1 and D_refl / D. One set serves every direction evaluated from wo (and
+// every lobe of the same roughness).
+struct WoTerms {
+    float nv, G1, D_refl_D;
+};
+OSLMI_HD WoTerms ggx_wo_terms(const GGX& d, V3 wo)
+{
+    WoTerms t;
+    t.nv       = vlength(V3(wo.x * d.ax, wo.y * d.ay, wo.z));
+    t.G1       = 2.0f * wo.z / (wo.z + t.nv);
+    t.D_refl_D = ggx_D_refl_D(d, wo);
+    return t;
 }
 // visible-normal sampling (Walter), used by the MiniMicrofacetGGX bake
 OSLMI_HD V3 ggx_sample_vndf(const GGX& d, V3 wo, float randu, float randv)
@@ -316,25 +325,34 @@ OSLMI_HD float interpolate_emiss(const float* E, int Nf, float roughness, float 
     return LERP(ff, LERP(rf, E[(fa * kNr + ra) * kNc + i], E[(fa * kNr + rb) * kNc + i]),
                 LERP(rf, E[(fb * kNr + ra) * kNc + i], E[(fb * kNr + rb) * kNc + i]));
 }
-// TabulatedEnergyCurve::Emiss_eval on table `table` of the table set
+// The table interval of a cosine: the first i in 1..15 with c < cosine i,
+// 15 if there is none (NaN included). Computed and corrected by one step
+// instead of searched: a search runs as long as its slowest lane, 15 rounds
+// of a wave in nearly every call.
+OSLMI_HD int cosine_interval(int table, float c)
+{
+    const float x = table == kLutMiniGGX ? sqrtf(smax(c, 0.0f)) : c;
+    int i         = static_cast<int>(smax(bmin(x * 15.0f, 14.0f), 0.0f)) + 1;
+    if (i > 1 && c < get_cosine(table, i - 1))
+        i--;
+    if (i < kNc - 1 && !(c < get_cosine(table, i)))
+        i++;
+    return i;
+}
+// TabulatedEnergyCurve::Emiss_eval on table `table` of the table set: the
+// entries of the interval's two cosines, interpolated. At and below the
+// first cosine the interpolation factor is clamped to 0, at and above the
+// last to 1, which leaves that entry exactly.
 OSLMI_HD float emiss_eval(const float* tables, int table, float roughness, float fresnel_index,
                           float c)
 {
-    const float* E = tables + table;
-    const int Nf   = table == kLutMiniGGX ? 1 : kNfRefl;
-    float cos0     = get_cosine(table, 0);
-    if (c <= cos0)
-        return interpolate_emiss(E, Nf, roughness, fresnel_index, 0);
-    for (int i = 1; i < kNc; i++) {
-        const float cos1 = get_cosine(table, i);
-        if (c < cos1) {
-            float q = (c - cos0) / (cos1 - cos0);
-            return LERP(q, interpolate_emiss(E, Nf, roughness, fresnel_index, i - 1),
-                        interpolate_emiss(E, Nf, roughness, fresnel_index, i));
-        }
-        cos0 = cos1;
-    }
-    return interpolate_emiss(E, Nf, roughness, fresnel_index, kNc - 1);
+    const float* E   = tables + table;
+    const int Nf     = table == kLutMiniGGX ? 1 : kNfRefl;
+    const int i      = cosine_interval(table, c);
+    const float cos0 = get_cosine(table, i - 1), cos1 = get_cosine(table, i);
+    return LERP((c - cos0) / (cos1 - cos0),
+                interpolate_emiss(E, Nf, roughness, fresnel_index, i - 1),
+                interpolate_emiss(E, Nf, roughness, fresnel_index, i));
 }
 
 // ---- Fresnel ------------------------------------------------------------
@@ -364,8 +382,8 @@ OSLMI_HD float dfresnel_table_index(float eta)
 }
 
 // microfacet reflection state of the two MTX microfacet lobes: GGX,
-// Fresnel (kind 0 dielectric, 1 generalized Schlick) and the
-// MiniMicrofacetGGX multiple-scattering energy E_ms of the lobe's
+// Fresnel (kind 0 dielectric, 1 generalized Schlick) and the factor msf of
+// the MiniMicrofacetGGX multiple-scattering energy E_ms of the lobe's
 // DielectricBSDF
 struct Spec {
     GGX d;
@@ -373,7 +391,7 @@ struct Spec {
     float eta;
     V3 F0, F90;
     float exponent, tir_cos;
-    float E_ms;
+    float msf;  // E_ms / max(0.01, 1 - E_ms)
     OSLMI_DEV V3 fresnel(float c) const
     {
         if (kind == 0)
@@ -388,7 +406,7 @@ struct Spec {
 struct SpecDielectric {
     GGX d;
     float eta;
-    float E_ms;
+    float msf;
     OSLMI_HD V3 fresnel(float c) const { return V3(dielectric_fresnel(eta, c)); }
 };
 
@@ -408,29 +426,50 @@ OSLMI_HD Sample zero_sample()
     return s;
 }
 
-// eval_turquin_microms_reflection (microfacet_tools_impl.h:345-378)
-template<class S> OSLMI_HD Sample eval_turquin(const S& sp, V3 wo, V3 wi)
+OSLMI_HD float ms_factor(float E_ms) { return E_ms / smax(0.01f, 1 - E_ms); }
+
+// eval_turquin_microms_reflection (microfacet_tools_impl.h:345-378) in two
+// parts: the geometry, which lobes of one roughness evaluated at one
+// direction share, and a lobe's weight.
+struct Refl {
+    bool on;  // both directions above the surface
+    V3 wi;
+    float cosMO, out, pdf;
+};
+OSLMI_HD Refl turquin_geometry(const GGX& d, const WoTerms& t, V3 wo, V3 wi)
 {
-    const float cosNO = wo.z;
-    const float cosNI = wi.z;
-    if (cosNI <= 0 || cosNO <= 0)
+    Refl r;
+    r.wi = wi;
+    r.on = !(wi.z <= 0 || wo.z <= 0);
+    if (!r.on) {
+        r.cosMO = r.out = r.pdf = 0.0f;
+        return r;
+    }
+    const V3 m     = normalized(wo + wi);
+    r.cosMO        = vdot(m, wo);
+    const float D  = ggx_D(d, m);
+    const float nl = vlength(V3(wi.x * d.ax, wi.y * d.ay, wi.z));
+    r.pdf          = (t.D_refl_D * D) / (4 * wo.z);
+    // G2 / G1 of the stretched directions
+    const float G2_G1 = wi.z * (wo.z + t.nv) / (wo.z * nl + wi.z * t.nv);
+    r.out             = G2_G1 * t.G1 / t.D_refl_D;
+    return r;
+}
+template<class S> OSLMI_HD Sample turquin_weight(const S& sp, const Refl& r)
+{
+    if (!r.on)
         return zero_sample();
-    V3 m            = normalized(wo + wi);
-    float cosMO     = vdot(m, wo);
-    const float D   = ggx_D(sp.d, m);
-    float D_refl_D  = ggx_D_refl_D(sp.d, wo);
-    float D_refl    = D_refl_D * D;
-    const float G1  = ggx_G1(sp.d, wo);
-    float pdf       = D_refl / (4 * cosNO);
-    const float out = ggx_G2_G1(sp.d, wi, wo) * G1 / D_refl_D;
-    const V3 F      = sp.fresnel(cosMO);
-    const float msf = sp.E_ms / smax(0.01f, 1 - sp.E_ms);
+    const V3 F = sp.fresnel(r.cosMO);
     Sample s;
-    s.wi        = wi;
-    s.weight    = (F * out) * (V3(1.0f) + F * msf);
-    s.pdf       = pdf;
+    s.wi        = r.wi;
+    s.weight    = (F * r.out) * (V3(1.0f) + F * sp.msf);
+    s.pdf       = r.pdf;
     s.roughness = -1.0f;
     return s;
+}
+template<class S> OSLMI_HD Sample eval_turquin(const S& sp, V3 wo, V3 wi)
+{
+    return turquin_weight(sp, turquin_geometry(sp.d, ggx_wo_terms(sp.d, wo), wo, wi));
 }
 
 // ---- sheen (Conty-Kulla) --------------------------------------------------
@@ -533,7 +572,7 @@ OSLMI_DEV void mx_micro(MxLobe* M, int kind, V3 N, V3 U, V3 refl_tint, float rou
         M->sp.tir_cos  = M->sp.eta >= 1 ? 0 : sqrtf(1 - SQR(M->sp.eta));
     }
     M->sp.d    = ggx_make(rough, aniso, rx < ry);
-    M->sp.E_ms = emiss_eval(T, kLutMiniGGX, rough, 0.0f, cosNO);
+    M->sp.msf  = ms_factor(emiss_eval(T, kLutMiniGGX, rough, 0.0f, cosNO));
     M->E = M->dorefl ? emiss_eval(T, kLutReflFront, rough, dfresnel_table_index(M->sp.eta), cosNO)
                      : 0.0f;
 }
