@@ -456,6 +456,13 @@ int oslmi_surrogate_grads(oslmi_surrogate* s, int64_t batch, const float* d_quer
 int oslmi_surrogate_train_step(oslmi_surrogate* s, int64_t batch, const float* d_query,
                                const float* d_target, float lr, float beta1, float beta2,
                                float eps, int step, void* stream);
+/* The same step on a minibatch drawn from n samples (d_query and d_target
+ * with leading dimension n): sample k is column d_index[k], each index in
+ * [0, n) (device, batch of them). */
+int oslmi_surrogate_train_step_indexed(oslmi_surrogate* s, int64_t batch, int64_t n,
+                                       const float* d_query, const float* d_target,
+                                       const int64_t* d_index, float lr, float beta1, float beta2,
+                                       float eps, int step, void* stream);
 /* Routing table: 64 cells (8 coat-roughness bins x 8 bins of the cosine
  * between L and the mirror direction of V); a non-zero cell sends its
  * queries to the exact closure. */

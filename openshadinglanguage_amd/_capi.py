@@ -72,6 +72,9 @@ def _declare(L):
         "oslmi_surrogate_grads": ([P, I64, P, P, P, P], I),
         "oslmi_surrogate_train_step": ([P, I64, P, P, ctypes.c_float, ctypes.c_float,
                                         ctypes.c_float, ctypes.c_float, I, P], I),
+        "oslmi_surrogate_train_step_indexed": ([P, I64, I64, P, P, P, ctypes.c_float,
+                                                ctypes.c_float, ctypes.c_float, ctypes.c_float, I,
+                                                P], I),
         "oslmi_surrogate_set_routing": ([P, P, I], I),
         "oslmi_surrogate_set_spot_check": ([P, ctypes.c_float], I),
         "oslmi_surrogate_infer": ([P, P, I64, P, P, P, P, P], I),

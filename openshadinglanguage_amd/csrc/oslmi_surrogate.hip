@@ -8,12 +8,12 @@
 // Outputs (4): log of the eval weight rgb and log pdf, normalised by
 // (y - mean) / std.
 //
-// Training (one step = one minibatch): row-major bf16 activations feed a
-// generic C = A B^T GEMM kernel (one wave per 16x16 tile, K in steps of 32,
-// split-K partials for the weight gradients); elementwise kernels add
-// biases, apply SiLU and its derivative, form the loss gradient and
-// transpose through LDS; Adam updates FP32 master weights and refreshes
-// the bf16 copies. All reductions run in a fixed order, so training is
+// Training (one step = one minibatch): one kernel takes 128 samples a
+// workgroup through the forward pass, the loss and the backward pass with
+// the activations in registers (MFMA operands chained layer to layer, see
+// k_fwd_bwd), and writes one partial gradient per workgroup; a second one
+// sums the partials in a fixed order, applies Adam to the FP32 master
+// weights and refreshes the packed bf16 copies. No atomics: training is
 // deterministic.
 //
 // Inference: one fused kernel. Each wave keeps every weight fragment in the
@@ -54,8 +54,8 @@ constexpr int OFF_B[6] = { 0, 2048, 6208, 10368, 14528, 16640 };
 constexpr int LAYER_OUT[6] = { 0, H, H, H, H, NOUT_PAD };
 constexpr int LAYER_IN[6]  = { 0, NIN_PAD, H, H, H, H };
 constexpr int NPARAM       = 16672;
-constexpr int EW_ROWS      = 64;    // samples per elementwise block
-constexpr int KCHUNK       = 2048;  // samples per split-K partial
+constexpr int TRAIN_ROWS   = 128;   // samples per training workgroup
+constexpr int BATCH_STEP   = 2048;  // max_batch comes in multiples of this
 
 struct Norm {
     float in_off[NIN], in_scale[NIN];
@@ -67,280 +67,320 @@ struct Domain {
     float lo[9], hi[9];  // coat ior, coat roughness, sheen roughness, F0 rgb, F90 rgb
 };
 
-__device__ __forceinline__ float silu(float z) { return z / (1.0f + expf(-z)); }
-__device__ __forceinline__ float dsilu(float z)
+// Hidden feature order along K of the packed fragments of layers 2 to 5: K
+// step s, lane group g, slot j holds feature 16 (2s + j/4) + 4g + j%4, which
+// is where the previous layer's accumulators left it.
+__host__ __device__ inline int hidden_k(int s, int g, int j)
 {
-    const float s = 1.0f / (1.0f + expf(-z));
-    return s * (1.0f + z * (1.0f - s));
+    return 16 * (2 * s + j / 4) + 4 * g + (j % 4);
 }
 
-// ---- training kernels --------------------------------------------------
-// C[m][n] = sum_k A[m][k] B[n][k]; A, B bf16 with K contiguous; one wave
-// per 16x16 tile; blockIdx.z selects a K chunk whose partial sum goes to
-// C + z * cstride. M, N multiples of 16, K and kchunk multiples of 32, lda
-// and ldb multiples of 8.
-__global__ __launch_bounds__(64) void k_gemm_nt(int K, const bf16* __restrict__ A, int lda,
-                                                const bf16* __restrict__ B, int ldb,
-                                                float* __restrict__ C, int ldc, int kchunk,
-                                                int64_t cstride)
+// ---- training ----------------------------------------------------------
+// Weights as MFMA A operands (bf16, 8 per lane, stored [fragment][lane][8]):
+//   forward, rows = outputs: W1 4 tiles; W2..W4 4 tiles x 2 K steps; W5 the
+//   16 rows that hold the outputs x 2 K steps; K in hidden_k order;
+//   backward, rows = inputs, K = outputs: W5 4 tiles x 1 K step (outputs
+//   beyond 32 do not exist); W4..W2 4 tiles x 2 K steps.
+constexpr int FWD_OF[6] = { 0, 0, 4, 12, 20, 28 }, NFWD = 30;
+constexpr int BWD_OF[6] = { 0, 0, 20, 12, 4, 0 }, NBWD = 28;
+
+__device__ __forceinline__ int layer_of(int p)
 {
-    const int lane = threadIdx.x;
-    const int r = lane & 15, g = lane >> 4;
-    const int m0 = blockIdx.y * 16, n0 = blockIdx.x * 16;
-    const int kb = blockIdx.z * kchunk;
-    const int ke = kb + kchunk < K ? kb + kchunk : K;
-    const bf16* a = A + (int64_t)(m0 + r) * lda + 8 * g;
-    const bf16* b = B + (int64_t)(n0 + r) * ldb + 8 * g;
-    f32x4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
-    for (int k = kb; k < ke; k += 32) {
-        const bf16x8 av = *reinterpret_cast<const bf16x8*>(a + k);
-        const bf16x8 bv = *reinterpret_cast<const bf16x8*>(b + k);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc, 0, 0, 0);
+    int l = 1;
+    while (l < 5 && p >= OFF_W[l + 1])
+        l++;
+    return l;
+}
+
+// Writes weight p = W[l][o][i] into its place in the two fragment sets.
+__device__ __forceinline__ void pack_weight(int l, int o, int i, float w, bf16* __restrict__ fwd,
+                                            bf16* __restrict__ bwd)
+{
+    const bf16 h = (bf16)w;
+    if (l < 5 || o < 16) {
+        const int s = l == 1 ? 0 : i >> 5, g = l == 1 ? i >> 3 : (i & 15) >> 2;
+        const int j = l == 1 ? i & 7 : 4 * ((i >> 4) & 1) + (i & 3);
+        const int f = FWD_OF[l] + (l == 1 ? o >> 4 : (l == 5 ? s : 2 * (o >> 4) + s));
+        fwd[(f * 64 + 16 * g + (o & 15)) * 8 + j] = h;
     }
-    float* c = C + blockIdx.z * cstride;
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-        c[(int64_t)(m0 + 4 * g + j) * ldc + n0 + r] = acc[j];
+    if (l > 1) {
+        const int s = o >> 5, g = (o & 15) >> 2, j = 4 * ((o >> 4) & 1) + (o & 3);
+        const int f = BWD_OF[l] + (l == 5 ? i >> 4 : 2 * (i >> 4) + s);
+        bwd[(f * 64 + 16 * g + (i & 15)) * 8 + j] = h;
+    }
 }
 
-// Normalised inputs X [B][32] and X^T [32][B] (bf16, zero padded) and
-// normalised log targets Y [B][4] from query planes q [14][ldq] and exact
-// outputs t [4][ldq] (weight rgb, pdf).
-__global__ __launch_bounds__(256) void k_prep(int B, Norm nm, const float* __restrict__ q,
-                                              const float* __restrict__ t, int64_t ldq,
-                                              bf16* __restrict__ X, bf16* __restrict__ XT,
-                                              float* __restrict__ Y)
+__global__ __launch_bounds__(256) void k_pack_train(const float* __restrict__ P,
+                                                    bf16* __restrict__ fwd, bf16* __restrict__ bwd)
 {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= B)
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= NPARAM)
         return;
-#pragma unroll
-    for (int k = 0; k < NIN_PAD; k++) {
-        float v = 0.0f;
-        if (k < NIN)
-            v = (q[k * ldq + s] - nm.in_off[k]) * nm.in_scale[k];
-        const bf16 h = (bf16)v;
-        X[(int64_t)s * NIN_PAD + k] = h;
-        XT[(int64_t)k * B + s]      = h;
-    }
-    if (t) {
-#pragma unroll
-        for (int o = 0; o < NOUT; o++) {
-            const float raw = t[o * ldq + s];
-            const float y   = o < 3 ? logf(fmaxf(raw, 1e-6f)) : logf(fmaxf(raw, 1e-12f));
-            Y[(int64_t)s * NOUT + o] = (y - nm.out_mu[o]) / nm.out_sd[o];
-        }
+    const int l = layer_of(p);
+    if (p < OFF_B[l]) {
+        const int e = p - OFF_W[l];
+        pack_weight(l, e / LAYER_IN[l], e % LAYER_IN[l], P[p], fwd, bwd);
     }
 }
 
-// Hidden layer epilogue over a block of 64 samples: Z += b, A = bf16(silu(Z)),
-// A^T through LDS.
-__global__ __launch_bounds__(256) void k_bias_silu(int B, float* __restrict__ Z,
-                                                   const float* __restrict__ bias,
-                                                   bf16* __restrict__ A, bf16* __restrict__ AT)
+// SiLU and its derivative from one sigmoid. exp2 and reciprocal are the
+// hardware's, about 1 ulp each; the activations are rounded to bf16 next.
+__device__ __forceinline__ void silu_both(float z, float* a, float* da)
 {
-    __shared__ bf16 tile[EW_ROWS][H + 2];
-    const int s0 = blockIdx.x * EW_ROWS;
-    for (int e = threadIdx.x; e < EW_ROWS * H; e += blockDim.x) {
-        const int s = e / H, o = e % H;
-        const int64_t idx = (int64_t)(s0 + s) * H + o;
-        const float z = Z[idx] + bias[o];
-        Z[idx]        = z;
-        const bf16 a  = (bf16)silu(z);
-        A[idx]        = a;
-        tile[s][o]    = a;
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < EW_ROWS * H; e += blockDim.x) {
-        const int o = e / EW_ROWS, s = e % EW_ROWS;
-        AT[(int64_t)o * B + s0 + s] = tile[s][o];
-    }
+    const float s = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * z));
+    *a            = z * s;
+    *da           = s * (1.0f + z * (1.0f - s));
 }
 
-// Output layer and loss: pred = Z5 + b5 (4 outputs), dZ5 = 2 (pred - Y) / (4B)
-// as bf16 [B][32] and [32][B]; bias-gradient and loss partials per block.
-__global__ __launch_bounds__(256) void k_loss(int B, const float* __restrict__ Z5,
-                                              const float* __restrict__ b5,
-                                              const float* __restrict__ Y,
-                                              bf16* __restrict__ dZ, bf16* __restrict__ dZT,
-                                              float* __restrict__ bpart,
-                                              float* __restrict__ lpart)
+// Sum over the 16 lanes of a row, in every one of them.
+__device__ __forceinline__ float row_sum(float v)
 {
-    __shared__ float red[NOUT_PAD][EW_ROWS + 1];
-    __shared__ float lred[EW_ROWS];
-    const int s0 = blockIdx.x * EW_ROWS;
-    for (int e = threadIdx.x; e < EW_ROWS * NOUT_PAD; e += blockDim.x) {
-        const int s = e / NOUT_PAD, o = e % NOUT_PAD;
-        float d = 0.0f;
-        if (o < NOUT) {
-            const float pred = Z5[(int64_t)(s0 + s) * NOUT_PAD + o] + b5[o];
-            d = pred - Y[(int64_t)(s0 + s) * NOUT + o];
+#define OSLMI_ROW_ADD(ctrl)                                                                    \
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, true));
+    OSLMI_ROW_ADD(0x121)  // row_ror:1, 2, 4, 8
+    OSLMI_ROW_ADD(0x122)
+    OSLMI_ROW_ADD(0x124)
+    OSLMI_ROW_ADD(0x128)
+#undef OSLMI_ROW_ADD
+    return v;
+}
+
+// Forward, loss and backward of 128 samples per workgroup; eight waves of 16
+// samples (the columns of a 16-wide MFMA tile; lane = 16 g + r holds sample
+// r). A layer is acc = W h with the weights as A operand and the samples as
+// columns: the accumulators (4 consecutive features of a sample per tile of
+// 16) are the next layer's B operand in place, forward and backward, so
+// activations never leave the registers. Only the weight gradients, which
+// contract over samples, need them across lanes: A^T and dZ^T of one layer
+// go through LDS ([feature][sample], double buffered, one barrier a layer),
+// and each wave accumulates half of 16 gradient rows.
+// The pass of one workgroup is a chain of latencies, not of bytes or flops.
+// Measured at a batch of 16384: 21.8 us here plus 4.5 us for k_reduce_adam,
+// against 240 us of the former form (22 launches of one-wave GEMM tiles and
+// elementwise kernels, every activation through memory four times); four
+// waves of 32 samples instead of eight of 16 took 28.4 us.
+// idx (optional): sample k of the batch is column idx[k] of the planes (one
+// outside them counts as no sample). part: [workgroup][NPARAM] partial
+// gradients; lpart: [workgroup] sums of squared errors.
+constexpr int LDT         = TRAIN_ROWS + 8;  // row pitch: conflict-free 16-byte reads
+constexpr int TRAIN_WAVES = TRAIN_ROWS / 16;
+__global__ __launch_bounds__(64 * TRAIN_WAVES) void k_fwd_bwd(
+    int B, Norm nm, const float* __restrict__ q, const float* __restrict__ t, int64_t ldq,
+    const int64_t* __restrict__ idx, const float* __restrict__ P, const bf16x8* __restrict__ fwd,
+    const bf16x8* __restrict__ bwd, float* __restrict__ part, float* __restrict__ lpart)
+{
+    __shared__ __align__(16) bf16 s_z[2][H][LDT], s_a[2][H][LDT];
+    __shared__ float s_b[TRAIN_WAVES][4 * H + 16], s_l[TRAIN_WAVES];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int g = lane >> 4, r = lane & 15;
+    const int col = wv * 16 + r;  // this lane's column of the workgroup's 128
+    float* pw     = part + (int64_t)blockIdx.x * NPARAM;
+    const int smp = blockIdx.x * TRAIN_ROWS + col;
+    bool live     = smp < B;
+    int64_t src   = live ? (idx ? idx[smp] : smp) : 0;
+    if (src < 0 || src >= ldq) {
+        live = false;
+        src  = 0;
+    }
+    bf16x8 x;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const int k   = 8 * g + j;
+        const int kc  = k < NIN ? k : 0;
+        const float v = (q[kc * ldq + src] - nm.in_off[kc]) * nm.in_scale[kc];
+        x[j]          = (bf16)(k < NIN && live ? v : 0.0f);
+    }
+    float raw[NOUT];
+#pragma unroll
+    for (int o = 0; o < NOUT; o++)
+        raw[o] = t[o * ldq + src];
+    // forward: h[l] layer l's activations (B operands), d[l] SiLU'
+    bf16x8 h[5][2];
+    f32x4 d[5][4];
+#pragma unroll
+    for (int l = 1; l <= 4; l++) {
+        f32x4 acc[4];
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+            const f32x4 b = *reinterpret_cast<const f32x4*>(P + OFF_B[l] + 16 * m + 4 * g);
+            if (l == 1) {
+                acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fwd[(FWD_OF[1] + m) * 64 + lane],
+                                                                 x, b, 0, 0, 0);
+            } else {
+                acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    fwd[(FWD_OF[l] + 2 * m) * 64 + lane], h[l - 1][0], b, 0, 0, 0);
+                acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    fwd[(FWD_OF[l] + 2 * m + 1) * 64 + lane], h[l - 1][1], acc[m], 0, 0, 0);
+            }
         }
-        red[o][s] = d;
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                float a, da;
+                silu_both(acc[m][j], &a, &da);
+                h[l][m >> 1][4 * (m & 1) + j] = (bf16)a;
+                d[l][m][j]                    = da;
+            }
     }
-    __syncthreads();
-    if (threadIdx.x < EW_ROWS) {
-        const int s = threadIdx.x;
-        float l = 0.0f;
-        for (int o = 0; o < NOUT; o++)
-            l += red[o][s] * red[o][s];
-        lred[s] = l;
-    }
-    __syncthreads();
+    // output layer, loss, and its gradient 2 (pred - y) / (4 B): lanes of
+    // group 0 hold the four outputs
+    f32x4 out = *reinterpret_cast<const f32x4*>(P + OFF_B[5] + 4 * g);
+    out = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fwd[FWD_OF[5] * 64 + lane], h[4][0], out, 0, 0, 0);
+    out = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fwd[(FWD_OF[5] + 1) * 64 + lane], h[4][1], out, 0, 0, 0);
     const float scale = 2.0f / (4.0f * (float)B);
-    for (int e = threadIdx.x; e < EW_ROWS * NOUT_PAD; e += blockDim.x) {
-        const int s = e / NOUT_PAD, o = e % NOUT_PAD;
-        const float g = red[o][s] * scale;
-        red[o][s]     = g;
-        dZ[(int64_t)(s0 + s) * NOUT_PAD + o] = (bf16)g;
+    float lsum = 0.0f;
+    bf16x8 z[2];  // dZ of the layer as B operand
+#pragma unroll
+    for (int o = 0; o < 4; o++) {
+        const float y = (logf(fmaxf(raw[o], o < 3 ? 1e-6f : 1e-12f)) - nm.out_mu[o]) / nm.out_sd[o];
+        const float e = g == 0 && live ? out[o] - y : 0.0f;
+        lsum += e * e;
+        z[0][o]       = (bf16)(e * scale);
+        z[0][4 + o]   = (bf16)0.0f;
+        z[1][o]       = (bf16)0.0f;
+        z[1][4 + o]   = (bf16)0.0f;
+        const float b = row_sum(e * scale);
+        if (r == 0)
+            s_b[wv][4 * H + 4 * g + o] = b;
+    }
+    lsum = row_sum(lsum);
+    if (lane == 0)
+        s_l[wv] = lsum;
+    // backward
+#pragma unroll
+    for (int l = 5; l >= 1; l--) {
+        const int buf = l & 1;
+        // dZ^T (the 16 rows of tile 0 for the output layer) and A^T
+#pragma unroll
+        for (int m = 0; m < (l == 5 ? 1 : 4); m++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                s_z[buf][16 * m + 4 * g + j][col] = z[m >> 1][4 * (m & 1) + j];
+        if (l > 1) {
+#pragma unroll
+            for (int m = 0; m < 4; m++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    s_a[buf][16 * m + 4 * g + j][col] = h[l - 1][m >> 1][4 * (m & 1) + j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                s_a[buf][8 * g + j][col] = x[j];
+        }
+        __syncthreads();
+        // the next layer's dZ, which needs no other wave
+        bf16x8 zn[2];
+        if (l > 1) {
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+                const int f = BWD_OF[l] + (l == 5 ? m : 2 * m);
+                f32x4 acc   = { 0.0f, 0.0f, 0.0f, 0.0f };
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bwd[f * 64 + lane], z[0], acc, 0, 0, 0);
+                if (l < 5)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bwd[(f + 1) * 64 + lane], z[1], acc, 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float v                  = acc[j] * d[l - 1][m][j];
+                    zn[m >> 1][4 * (m & 1) + j] = (bf16)v;
+                    const float b = row_sum(v);
+                    if (r == 0)
+                        s_b[wv][(l - 2) * H + 16 * m + 4 * g + j] = b;
+                }
+            }
+        }
+        // weight gradient: rows = outputs (dZ), columns = inputs (A). Waves w
+        // and w + 4 share a row tile; the output layer has one row tile, whose
+        // four column tiles go to waves 0 to 3.
+        const int nin = LAYER_IN[l];
+        if (l < 5 || wv < 4) {
+            const int rt = l == 5 ? 0 : wv & 3;
+            bf16x8 zr[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                zr[k] = *reinterpret_cast<const bf16x8*>(&s_z[buf][16 * rt + r][32 * k + 8 * g]);
+            constexpr int kTiles[6] = { 0, 1, 2, 2, 2, 1 };
+#pragma unroll
+            for (int ct = 0; ct < kTiles[l]; ct++) {
+                const int c0 = 16 * (l == 5 ? wv : kTiles[l] * (wv >> 2) + ct);
+                f32x4 acc    = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        zr[k], *reinterpret_cast<const bf16x8*>(&s_a[buf][c0 + r][32 * k + 8 * g]), acc,
+                        0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    pw[OFF_W[l] + (16 * rt + 4 * g + j) * nin + c0 + r] = acc[j];
+            }
+        }
+        z[0] = zn[0];
+        z[1] = zn[1];
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < EW_ROWS * NOUT_PAD; e += blockDim.x) {
-        const int o = e / EW_ROWS, s = e % EW_ROWS;
-        dZT[(int64_t)o * B + s0 + s] = (bf16)red[o][s];
-    }
-    if (threadIdx.x < NOUT_PAD) {
-        const int o = threadIdx.x;
-        float acc = 0.0f;
-        for (int s = 0; s < EW_ROWS; s++)
-            acc += red[o][s];
-        bpart[(int64_t)blockIdx.x * NOUT_PAD + o] = acc;
+    // bias gradients and the loss: the waves' sums in order
+    for (int k = threadIdx.x; k < 4 * H + 16; k += blockDim.x) {
+        float b = s_b[0][k];
+#pragma unroll
+        for (int w = 1; w < TRAIN_WAVES; w++)
+            b += s_b[w][k];
+        pw[k < 4 * H ? OFF_B[1 + k / H] + k % H : OFF_B[5] + k - 4 * H] = b;
     }
     if (threadIdx.x == 0) {
-        float acc = 0.0f;
-        for (int s = 0; s < EW_ROWS; s++)
-            acc += lred[s];
-        lpart[blockIdx.x] = acc;
+        float e = s_l[0];
+#pragma unroll
+        for (int w = 1; w < TRAIN_WAVES; w++)
+            e += s_l[w];
+        lpart[blockIdx.x] = e;
     }
 }
 
-// Hidden layer backward epilogue: dZ = dA * silu'(Z) as bf16 [B][64] and
-// [64][B]; bias-gradient partials per block.
-__global__ __launch_bounds__(256) void k_silu_bwd(int B, const float* __restrict__ dA,
-                                                  const float* __restrict__ Z,
-                                                  bf16* __restrict__ dZ, bf16* __restrict__ dZT,
-                                                  float* __restrict__ bpart)
+struct AdamArgs {
+    float lr, b1, b2, eps, bc1, bc2;
+};
+
+// Sums every parameter's nb partials (64 parameters and four segments of
+// the partials per workgroup, fixed order) into G and, with update, applies
+// Adam to the FP32 master weights and refreshes the packed bf16 weights. The
+// padding outputs 16..31 of the last layer have no partials: gradient zero.
+__global__ __launch_bounds__(256) void k_reduce_adam(const float* __restrict__ part, int nb,
+                                                     float* __restrict__ G, int update, AdamArgs ad,
+                                                     float* __restrict__ P, float* __restrict__ Mm,
+                                                     float* __restrict__ Vv, bf16* __restrict__ fwd,
+                                                     bf16* __restrict__ bwd)
 {
-    __shared__ float tile[EW_ROWS][H + 1];
-    const int s0 = blockIdx.x * EW_ROWS;
-    for (int e = threadIdx.x; e < EW_ROWS * H; e += blockDim.x) {
-        const int s = e / H, o = e % H;
-        const int64_t idx = (int64_t)(s0 + s) * H + o;
-        const float g     = dA[idx] * dsilu(Z[idx]);
-        tile[s][o]        = g;
-        dZ[idx]           = (bf16)g;
+    __shared__ float s_seg[4][64];
+    const int e = threadIdx.x & 63, seg = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + e;
+    const bool padding = (p >= OFF_W[5] + 16 * H && p < OFF_B[5]) || p >= OFF_B[5] + 16;
+    const int per = (nb + 3) / 4;
+    const int k1 = per * (seg + 1) < nb ? per * (seg + 1) : nb;
+    float sum = 0.0f;
+    if (p < NPARAM && !padding) {
+#pragma unroll 8
+        for (int k = per * seg; k < k1; k++)
+            sum += part[(int64_t)k * NPARAM + p];
     }
+    s_seg[seg][e] = sum;
     __syncthreads();
-    for (int e = threadIdx.x; e < EW_ROWS * H; e += blockDim.x) {
-        const int o = e / EW_ROWS, s = e % EW_ROWS;
-        dZT[(int64_t)o * B + s0 + s] = (bf16)tile[s][o];
-    }
-    if (threadIdx.x < H) {
-        const int o = threadIdx.x;
-        float acc = 0.0f;
-        for (int s = 0; s < EW_ROWS; s++)
-            acc += tile[s][o];
-        bpart[(int64_t)blockIdx.x * H + o] = acc;
-    }
-}
-
-// Reduces the gradient of every parameter (weight partials over split-K
-// chunks, bias partials over blocks, fixed order) into G. Weight partials
-// of layer l: [nsplit][out][in] at wpart + nsplit * OFF_W[l]; bias
-// partials: [nblk][out] at bpart + nblk * (l - 1) * H.
-__global__ __launch_bounds__(256) void k_reduce_grads(const float* __restrict__ wpart,
-                                                      const float* __restrict__ bpart,
-                                                      int nsplit, int nblk,
-                                                      float* __restrict__ G)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= NPARAM)
+    if (seg != 0 || p >= NPARAM)
         return;
-    int l = 1;
-    while (l < 5 && p >= OFF_W[l + 1])
-        l++;
-    const int nw = LAYER_OUT[l] * LAYER_IN[l];
-    if (p >= OFF_B[l])
-        return;  // biases: k_reduce_bias
-    float g = 0.0f;
-    const int e = p - OFF_W[l];
-    const float* slab = wpart + (int64_t)nsplit * OFF_W[l];
-    for (int k = 0; k < nsplit; k++)
-        g += slab[(int64_t)k * nw + e];
-    G[p] = g;
-}
-
-// Bias gradients: one wave per bias, each lane summing every 64th
-// per-block partial, then a fixed-order shuffle reduction (deterministic).
-__global__ __launch_bounds__(64) void k_reduce_bias(const float* __restrict__ bpart, int nblk,
-                                                    float* __restrict__ G)
-{
-    int l = 1, o = blockIdx.x;
-    while (l < 5 && o >= LAYER_OUT[l]) {
-        o -= LAYER_OUT[l];
-        l++;
-    }
-    const int nout    = LAYER_OUT[l];
-    const float* slab = bpart + (int64_t)nblk * (l - 1) * H;
-    float g = 0.0f;
-    for (int k = threadIdx.x; k < nblk; k += 64)
-        g += slab[(int64_t)k * nout + o];
-    for (int off = 32; off > 0; off >>= 1)
-        g += __shfl_down(g, off);
-    if (threadIdx.x == 0)
-        G[OFF_B[l] + o] = g;
-}
-
-// Adam on FP32 master weights; refreshes the bf16 W and W^T copies.
-__global__ __launch_bounds__(256) void k_adam(float* __restrict__ P, float* __restrict__ Mm,
-                                              float* __restrict__ Vv,
-                                              const float* __restrict__ G, float lr, float b1,
-                                              float b2, float eps, float bc1, float bc2,
-                                              bf16* __restrict__ Wb, bf16* __restrict__ WTb)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= NPARAM)
+    const float gr = ((s_seg[0][e] + s_seg[1][e]) + s_seg[2][e]) + s_seg[3][e];
+    G[p]           = gr;
+    if (!update)
         return;
-    const float g = G[p];
-    const float m = b1 * Mm[p] + (1.0f - b1) * g;
-    const float v = b2 * Vv[p] + (1.0f - b2) * g * g;
+    const float m = ad.b1 * Mm[p] + (1.0f - ad.b1) * gr;
+    const float v = ad.b2 * Vv[p] + (1.0f - ad.b2) * gr * gr;
     Mm[p]         = m;
     Vv[p]         = v;
-    const float w = P[p] - lr * (m / bc1) / (sqrtf(v / bc2) + eps);
+    const float w = P[p] - ad.lr * (m / ad.bc1) / (sqrtf(v / ad.bc2) + ad.eps);
     P[p]          = w;
-    int l = 1;
-    while (l < 5 && p >= OFF_W[l + 1])
-        l++;
+    const int l   = layer_of(p);
     if (p < OFF_B[l]) {
-        const int e = p - OFF_W[l];
-        const int o = e / LAYER_IN[l], i = e % LAYER_IN[l];
-        Wb[OFF_W[l] + e]                        = (bf16)w;
-        WTb[OFF_W[l] + i * LAYER_OUT[l] + o] = (bf16)w;
+        const int k = p - OFF_W[l];
+        pack_weight(l, k / LAYER_IN[l], k % LAYER_IN[l], w, fwd, bwd);
     }
 }
-
-__global__ void k_refresh_bf16(const float* __restrict__ P, bf16* __restrict__ Wb,
-                               bf16* __restrict__ WTb)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= NPARAM)
-        return;
-    int l = 1;
-    while (l < 5 && p >= OFF_W[l + 1])
-        l++;
-    if (p < OFF_B[l]) {
-        const int e = p - OFF_W[l];
-        const int o = e / LAYER_IN[l], i = e % LAYER_IN[l];
-        Wb[OFF_W[l] + e]                     = (bf16)P[p];
-        WTb[OFF_W[l] + i * LAYER_OUT[l] + o] = (bf16)P[p];
-    }
-}
-
-}  // namespace surrogate
-}  // namespace oslmi
-
-namespace oslmi {
-namespace surrogate {
 
 // ---- inference ---------------------------------------------------------
 // Packed fragments: 30 per lane (W1 4 tiles; W2..W4 4 tiles x 2 K steps;
@@ -353,14 +393,6 @@ struct InferConsts {
     Norm nm;
     Domain dom;
 };
-
-// Hidden feature order along K of the packed W2..W5 fragments: K step s,
-// lane group g, slot j holds feature 16 (2s + j/4) + 4g + j%4, which is
-// where the previous layer's accumulators left it.
-__host__ __device__ inline int hidden_k(int s, int g, int j)
-{
-    return 16 * (2 * s + j / 4) + 4 * g + (j % 4);
-}
 
 // SiLU for inference with the hardware exp2 and reciprocal (v_exp_f32,
 // v_rcp_f32, about 1 ulp each), on pre-activations scaled by -log2(e):
@@ -705,18 +737,10 @@ struct Context {
     float* Mm = nullptr;
     float* Vv = nullptr;
     float* G = nullptr;
-    bf16* Wb = nullptr;   // bf16 W (layer layouts as P)
-    bf16* WTb = nullptr;  // bf16 W^T
-    // activations / workspaces for max_batch samples
-    bf16 *X = nullptr, *XT = nullptr;
-    float* Y = nullptr;
-    float* Z[6] = {};
-    bf16 *A[5] = {}, *AT[5] = {};
-    bf16 *dZ = nullptr, *dZT = nullptr;
-    float* dA = nullptr;
-    float* wpart = nullptr;
-    float* bpart = nullptr;
-    float* lpart = nullptr;
+    bf16* fwd = nullptr;  // packed bf16 weights (training fragments)
+    bf16* bwd = nullptr;
+    float* part = nullptr;   // [workgroup][NPARAM] for max_batch samples
+    float* lpart = nullptr;  // [workgroup]
     // inference
     bf16x8* frag = nullptr;
     f32x4* biasp = nullptr;
@@ -728,29 +752,14 @@ struct Context {
 
 int ctx_alloc(Context* c)
 {
-    const int64_t B = c->max_batch;
-    const int64_t nsplit = (B + KCHUNK - 1) / KCHUNK;
-    const int64_t nblk   = B / EW_ROWS;
+    const int64_t nb = (c->max_batch + TRAIN_ROWS - 1) / TRAIN_ROWS;
     struct Item {
         void** p;
         size_t bytes;
     } items[] = {
         { (void**)&c->P, NPARAM * 4 }, { (void**)&c->Mm, NPARAM * 4 }, { (void**)&c->Vv, NPARAM * 4 },
-        { (void**)&c->G, NPARAM * 4 }, { (void**)&c->Wb, NPARAM * 2 }, { (void**)&c->WTb, NPARAM * 2 },
-        { (void**)&c->X, (size_t)B * NIN_PAD * 2 }, { (void**)&c->XT, (size_t)B * NIN_PAD * 2 },
-        { (void**)&c->Y, (size_t)B * NOUT * 4 },
-        { (void**)&c->Z[1], (size_t)B * H * 4 }, { (void**)&c->Z[2], (size_t)B * H * 4 },
-        { (void**)&c->Z[3], (size_t)B * H * 4 }, { (void**)&c->Z[4], (size_t)B * H * 4 },
-        { (void**)&c->Z[5], (size_t)B * NOUT_PAD * 4 },
-        { (void**)&c->A[1], (size_t)B * H * 2 }, { (void**)&c->A[2], (size_t)B * H * 2 },
-        { (void**)&c->A[3], (size_t)B * H * 2 }, { (void**)&c->A[4], (size_t)B * H * 2 },
-        { (void**)&c->AT[1], (size_t)B * H * 2 }, { (void**)&c->AT[2], (size_t)B * H * 2 },
-        { (void**)&c->AT[3], (size_t)B * H * 2 }, { (void**)&c->AT[4], (size_t)B * H * 2 },
-        { (void**)&c->dZ, (size_t)B * H * 2 }, { (void**)&c->dZT, (size_t)B * H * 2 },
-        { (void**)&c->dA, (size_t)B * H * 4 },
-        { (void**)&c->wpart, (size_t)nsplit * NPARAM * 4 },
-        { (void**)&c->bpart, (size_t)nblk * 5 * H * 4 },
-        { (void**)&c->lpart, (size_t)nblk * 4 },
+        { (void**)&c->G, NPARAM * 4 }, { (void**)&c->fwd, NFWD * 64 * 16 }, { (void**)&c->bwd, NBWD * 64 * 16 },
+        { (void**)&c->part, (size_t)nb * NPARAM * 4 }, { (void**)&c->lpart, (size_t)nb * 4 },
         { (void**)&c->frag, (size_t)NFRAG * 64 * 16 }, { (void**)&c->biasp, (size_t)NBIAS * 64 * 16 },
     };
     for (auto& it : items) {
@@ -766,61 +775,24 @@ int ctx_alloc(Context* c)
 
 void ctx_free(Context* c)
 {
-    void* ptrs[] = { c->P, c->Mm, c->Vv, c->G, c->Wb, c->WTb, c->X, c->XT, c->Y, c->Z[1], c->Z[2],
-                     c->Z[3], c->Z[4], c->Z[5], c->A[1], c->A[2], c->A[3], c->A[4], c->AT[1],
-                     c->AT[2], c->AT[3], c->AT[4], c->dZ, c->dZT, c->dA, c->wpart, c->bpart,
-                     c->lpart, c->frag, c->biasp };
+    void* ptrs[] = { c->P, c->Mm, c->Vv, c->G, c->fwd, c->bwd, c->part, c->lpart, c->frag, c->biasp };
     for (void* p : ptrs)
         if (p)
             (void)hipFree(p);
 }
 
-static void gemm(hipStream_t st, int M, int N, int K, const bf16* A, int lda, const bf16* B,
-                 int ldb, float* C, int ldc, int kchunk, int64_t cstride)
-{
-    const int splits = (K + kchunk - 1) / kchunk;
-    hipLaunchKernelGGL(k_gemm_nt, dim3(N / 16, M / 16, splits), dim3(64), 0, st, K, A, lda, B, ldb,
-                       C, ldc, kchunk, cstride);
-}
-
 // Forward + backward over a batch of B samples (B a multiple of 64, at most
-// max_batch); leaves the reduced gradients in G and per-block loss partials.
-int fwd_bwd(Context* c, int64_t B64, const float* q, const float* t, int64_t ldq, hipStream_t st)
+// max_batch) and, with adam, the weight update; leaves the reduced gradients
+// in G and per-workgroup loss partials.
+int fwd_bwd(Context* c, int64_t B64, const float* q, const float* t, int64_t ldq, const int64_t* idx,
+            const AdamArgs* adam, hipStream_t st)
 {
-    const int B    = (int)B64;
-    const int nblk = B / EW_ROWS;
-    const int nsplit = (B + KCHUNK - 1) / KCHUNK;
-    hipLaunchKernelGGL(k_prep, dim3((B + 255) / 256), dim3(256), 0, st, B, c->nm, q, t, ldq, c->X,
-                       c->XT, c->Y);
-    // forward
-    const bf16* in = c->X;
-    int kin = NIN_PAD;
-    for (int l = 1; l <= 4; l++) {
-        gemm(st, B, H, kin, in, kin, c->Wb + OFF_W[l], kin, c->Z[l], H, kin, 0);
-        hipLaunchKernelGGL(k_bias_silu, dim3(nblk), dim3(256), 0, st, B, c->Z[l], c->P + OFF_B[l],
-                           c->A[l], c->AT[l]);
-        in  = c->A[l];
-        kin = H;
-    }
-    gemm(st, B, NOUT_PAD, H, c->A[4], H, c->Wb + OFF_W[5], H, c->Z[5], NOUT_PAD, H, 0);
-    hipLaunchKernelGGL(k_loss, dim3(nblk), dim3(256), 0, st, B, c->Z[5], c->P + OFF_B[5], c->Y,
-                       c->dZ, c->dZT, c->bpart + (int64_t)nblk * 4 * H, c->lpart);
-    // backward
-    for (int l = 5; l >= 1; l--) {
-        const int nout = LAYER_OUT[l], nin = LAYER_IN[l];
-        const bf16* inT = l == 1 ? c->XT : c->AT[l - 1];
-        gemm(st, nout, nin, B, c->dZT, B, inT, B, c->wpart + (int64_t)nsplit * OFF_W[l], nin,
-             KCHUNK, (int64_t)nout * nin);
-        if (l > 1) {
-            gemm(st, B, H, nout, c->dZ, nout, c->WTb + OFF_W[l], nout, c->dA, H, nout, 0);
-            hipLaunchKernelGGL(k_silu_bwd, dim3(nblk), dim3(256), 0, st, B, c->dA, c->Z[l - 1],
-                               c->dZ, c->dZT, c->bpart + (int64_t)nblk * (l - 2) * H);
-        }
-    }
-    hipLaunchKernelGGL(k_reduce_grads, dim3((NPARAM + 255) / 256), dim3(256), 0, st, c->wpart,
-                       c->bpart, nsplit, nblk, c->G);
-    hipLaunchKernelGGL(k_reduce_bias, dim3(4 * H + NOUT_PAD), dim3(64), 0, st, c->bpart, nblk,
-                       c->G);
+    const int B  = (int)B64;
+    const int nb = (B + TRAIN_ROWS - 1) / TRAIN_ROWS;
+    hipLaunchKernelGGL(k_fwd_bwd, dim3(nb), dim3(64 * TRAIN_WAVES), 0, st, B, c->nm, q, t, ldq, idx, c->P,
+                       (const bf16x8*)c->fwd, (const bf16x8*)c->bwd, c->part, c->lpart);
+    hipLaunchKernelGGL(k_reduce_adam, dim3((NPARAM + 63) / 64), dim3(256), 0, st, c->part, nb, c->G,
+                       adam ? 1 : 0, adam ? *adam : AdamArgs {}, c->P, c->Mm, c->Vv, c->fwd, c->bwd);
     return check_launch("surrogate fwd/bwd");
 }
 
@@ -909,7 +881,7 @@ struct oslmi_surrogate {
 
 extern "C" oslmi_surrogate* oslmi_surrogate_create(int64_t max_batch)
 {
-    if (max_batch < 64 || max_batch % KCHUNK != 0) {
+    if (max_batch < 64 || max_batch % BATCH_STEP != 0) {
         set_error(OSLMI_ERR_INVALID, "oslmi_surrogate_create: max_batch must be a positive "
                                      "multiple of 2048");
         return nullptr;
@@ -967,8 +939,8 @@ extern "C" int oslmi_surrogate_set_params(oslmi_surrogate* s, const float* param
         return rc;
     if (int rc = check_hip(hipMemset(s->c.Vv, 0, NPARAM * 4), "hipMemset"))
         return rc;
-    hipLaunchKernelGGL(k_refresh_bf16, dim3((NPARAM + 255) / 256), dim3(256), 0, 0, s->c.P,
-                       s->c.Wb, s->c.WTb);
+    hipLaunchKernelGGL(k_pack_train, dim3((NPARAM + 255) / 256), dim3(256), 0, 0, s->c.P,
+                       s->c.fwd, s->c.bwd);
     if (int rc = check_launch("oslmi_surrogate_set_params"))
         return rc;
     s->c.host_params.assign(params, params + NPARAM);
@@ -1003,13 +975,13 @@ extern "C" int oslmi_surrogate_grads(oslmi_surrogate* s, int64_t batch, const fl
         return rc;
     if (!d_target || !grads)
         return set_error(OSLMI_ERR_INVALID, "oslmi_surrogate_grads: null argument");
-    if (int rc = fwd_bwd(&s->c, batch, d_query, d_target, batch, 0))
+    if (int rc = fwd_bwd(&s->c, batch, d_query, d_target, batch, nullptr, nullptr, 0))
         return rc;
     if (int rc = check_hip(hipMemcpy(grads, s->c.G, NPARAM * 4, hipMemcpyDeviceToHost),
                            "hipMemcpy(grads)"))
         return rc;
     if (loss) {
-        std::vector<float> lp(batch / EW_ROWS);
+        std::vector<float> lp((batch + TRAIN_ROWS - 1) / TRAIN_ROWS);
         if (int rc = check_hip(hipMemcpy(lp.data(), s->c.lpart, lp.size() * 4,
                                          hipMemcpyDeviceToHost), "hipMemcpy(loss)"))
             return rc;
@@ -1021,6 +993,18 @@ extern "C" int oslmi_surrogate_grads(oslmi_surrogate* s, int64_t batch, const fl
     return OSLMI_OK;
 }
 
+static int train_step(oslmi_surrogate* s, int64_t batch, const float* q, const float* t, int64_t ldq,
+                      const int64_t* idx, float lr, float beta1, float beta2, float eps, int step,
+                      void* stream)
+{
+    AdamArgs ad { lr, beta1, beta2, eps, 1.0f - powf(beta1, (float)step),
+                  1.0f - powf(beta2, (float)step) };
+    if (int rc = fwd_bwd(&s->c, batch, q, t, ldq, idx, &ad, (hipStream_t)stream))
+        return rc;
+    s->c.packed = false;
+    return OSLMI_OK;
+}
+
 extern "C" int oslmi_surrogate_train_step(oslmi_surrogate* s, int64_t batch, const float* d_query,
                                           const float* d_target, float lr, float beta1,
                                           float beta2, float eps, int step, void* stream)
@@ -1029,15 +1013,19 @@ extern "C" int oslmi_surrogate_train_step(oslmi_surrogate* s, int64_t batch, con
         return rc;
     if (!d_target || step < 1)
         return set_error(OSLMI_ERR_INVALID, "oslmi_surrogate_train_step: bad argument");
-    hipStream_t st = (hipStream_t)stream;
-    if (int rc = fwd_bwd(&s->c, batch, d_query, d_target, batch, st))
+    return train_step(s, batch, d_query, d_target, batch, nullptr, lr, beta1, beta2, eps, step, stream);
+}
+
+extern "C" int oslmi_surrogate_train_step_indexed(oslmi_surrogate* s, int64_t batch, int64_t n,
+                                                  const float* d_query, const float* d_target,
+                                                  const int64_t* d_index, float lr, float beta1,
+                                                  float beta2, float eps, int step, void* stream)
+{
+    if (int rc = batch_ok(s, batch, d_query, "oslmi_surrogate_train_step_indexed"))
         return rc;
-    const float bc1 = 1.0f - powf(beta1, (float)step);
-    const float bc2 = 1.0f - powf(beta2, (float)step);
-    hipLaunchKernelGGL(k_adam, dim3((NPARAM + 255) / 256), dim3(256), 0, st, s->c.P, s->c.Mm,
-                       s->c.Vv, s->c.G, lr, beta1, beta2, eps, bc1, bc2, s->c.Wb, s->c.WTb);
-    s->c.packed = false;
-    return check_launch("oslmi_surrogate_train_step");
+    if (!d_target || !d_index || n < 1 || step < 1)
+        return set_error(OSLMI_ERR_INVALID, "oslmi_surrogate_train_step_indexed: bad argument");
+    return train_step(s, batch, d_query, d_target, n, d_index, lr, beta1, beta2, eps, step, stream);
 }
 
 extern "C" int oslmi_surrogate_set_routing(oslmi_surrogate* s, const unsigned char* cells,

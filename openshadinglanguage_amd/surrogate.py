@@ -138,27 +138,36 @@ class Surrogate:
         progress(k) (optional) is called every 2000 steps."""
         import torch
         n = queries.shape[1]
+        if (tuple(queries.shape) != (NIN, n) or targets.dim() != 2 or targets.shape[0] != NOUT
+                or targets.shape[1] < n):
+            raise ValueError("train needs queries [14, n] and targets [4, n]")
+        for x in (queries, targets):
+            if not x.is_cuda or x.dtype != torch.float32:
+                raise ValueError("train needs float32 CUDA tensors")
+        # the step reads whole planes of n values; other strides are copied once
+        queries, targets = queries.contiguous(), targets[:, :n].contiguous()
         gen = torch.Generator(device=queries.device)
         gen.manual_seed(seed)
-        qb = torch.empty((NIN, batch), device=queries.device)
-        tb = torch.empty((NOUT, batch), device=queries.device)
         stream = stream or torch.cuda.current_stream()
         sp = ctypes.c_void_p(stream.cuda_stream)
         t0 = time.perf_counter()
         log = []
-        for k in range(steps):
-            idx = torch.randint(0, n, (batch,), device=queries.device, generator=gen)
-            torch.index_select(queries, 1, idx, out=qb)
-            torch.index_select(targets, 1, idx, out=tb)
-            self.step += 1
-            cur = lr_min + 0.5 * (lr - lr_min) * (1 + math.cos(math.pi * k / max(1, steps)))
-            check(self.L.oslmi_surrogate_train_step(self.h, batch, _p(qb), _p(tb), cur, 0.9,
-                                                    0.999, 1e-8, self.step, sp))
-            if log_every and (k % log_every == 0 or k == steps - 1):
-                _, loss = self.grads(qb, tb)
-                log.append((k, loss))
-            if progress and k % 2000 == 0:
-                progress(k)
+        pq, pt = _p(queries), _p(targets)
+        with torch.cuda.stream(stream):
+            for k in range(steps):
+                idx = torch.randint(0, n, (batch,), device=queries.device, generator=gen)
+                self.step += 1
+                cur = lr_min + 0.5 * (lr - lr_min) * (1 + math.cos(math.pi * k / max(1, steps)))
+                check(self.L.oslmi_surrogate_train_step_indexed(
+                    self.h, batch, n, pq, pt, _p(idx), cur, 0.9, 0.999, 1e-8, self.step, sp))
+                if log_every and (k % log_every == 0 or k == steps - 1):
+                    qb = queries.index_select(1, idx)
+                    tb = targets.index_select(1, idx)
+                    stream.synchronize()  # grads runs on the null stream
+                    _, loss = self.grads(qb, tb)
+                    log.append((k, loss))
+                if progress and k % 2000 == 0:
+                    progress(k)
         torch.cuda.synchronize()
         return {"steps": steps, "batch": batch, "seconds": time.perf_counter() - t0, "log": log}
 
