@@ -97,8 +97,8 @@ void oslmi_shadingsys_destroy(oslmi_shadingsys* ss);
  * "closure_export" (0/1: they also export Ci's lobes, for
  * oslmi_execute_batch_closures), and
  * "gpu_waves_per_eu" (0..8: the occupancy, in waves per SIMD, the emitted
- * kernels are register-allocated for; default 6, 0 leaves it to the
- * compiler). */
+ * kernels are register-allocated for; 0 leaves it to the compiler; unset:
+ * 6, for kernels with MaterialX closures 3, with their export 2). */
 int oslmi_shadingsys_attribute(oslmi_shadingsys* ss, const char* name, const char* value);
 /* Named coordinate systems, the renderer services behind transform(),
  * matrix(space) and getmatrix(): RendererServices::get_matrix /

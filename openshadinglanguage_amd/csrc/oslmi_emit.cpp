@@ -50,14 +50,21 @@ std::string flit(float f)
     return buf;
 }
 
-// launch bounds of every emitted kernel (256 work-items per workgroup) and,
-// when the shading system sets one, the occupancy target the register
-// allocator works to
-std::string kernel_attributes(const ShadingSys& ss)
+// launch bounds of every emitted kernel (256 work-items per workgroup) and
+// the occupancy target (waves per SIMD) the register allocator works to: the
+// shading system's, or by what the kernel holds. MaterialX lobes carry about
+// 40 registers each and need 160 to 250 in all: at six waves they spill 640
+// bytes a work-item. Measured (us, the layered material over 262,147 points,
+// six / four / three / two waves): sampled 83.8 / 66.6 / 48.6 / 59.3,
+// evaluated 42.0 / 33.6 / 22.6 / 27.5, exported (21 parameters a lobe more)
+// 80.5 / 67.3 / 43.8 / 31.2. Kernels without them run best at six (layered3,
+// 1M points: 266 us; 278, 306, 301 at five, four, three).
+std::string kernel_attributes(const ShadingSys& ss, bool mx, bool exported)
 {
     std::string a = "__launch_bounds__(256)";
-    if (ss.waves_per_eu > 0)
-        a += " __attribute__((amdgpu_waves_per_eu(" + std::to_string(ss.waves_per_eu) + ")))";
+    const int w   = ss.waves_per_eu >= 0 ? ss.waves_per_eu : !mx ? 6 : exported ? 2 : 3;
+    if (w > 0)
+        a += " __attribute__((amdgpu_waves_per_eu(" + std::to_string(w) + ")))";
     return a;
 }
 
@@ -1650,7 +1657,7 @@ struct Emitter {
         std::ostringstream k;
         k << "// Emitted by the oslmi group emitter for group '" << g.name << "'.\n";
         k << prelude(uses_mx, g.can_export, uses_aniso);
-        k << "extern \"C\" __global__ " << kernel_attributes(ss) << " void oslmi_group_main(GroupArgs A)\n{\n";
+        k << "extern \"C\" __global__ " << kernel_attributes(ss, uses_mx, g.can_export) << " void oslmi_group_main(GroupArgs A)\n{\n";
         k << "    using Closure = LobeList<" << closure_capacity() << ">;\n";
         if (uses_cs)
             k << "    const ColorSysDev* CS = (const ColorSysDev*)A.colorsys;\n";
@@ -1755,7 +1762,7 @@ bool emit_batch(const ShadingSys& ss, const std::vector<Group*>& groups,
          "    if (threadIdx.x == 0) *s_tile = atomicAdd(counter, 1);\n"
          "    __syncthreads();\n"
          "    return *s_tile;\n}\n";
-    k << "extern \"C\" __global__ " << kernel_attributes(ss) << " void oslmi_batch_main(BatchArgs B)\n{\n";
+    k << "extern \"C\" __global__ " << kernel_attributes(ss, any_mx, false) << " void oslmi_batch_main(BatchArgs B)\n{\n";
     k << "    const GroupArgs* __restrict__ args = B.args;\n";
     k << "    __shared__ int s_tile;\n";
     if (any_bb) {

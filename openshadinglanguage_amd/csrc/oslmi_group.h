@@ -132,7 +132,7 @@ struct ShadingSys {
     std::string commonspace = "world";  // synonym of "common"
     std::string cache_dir;   // code-object cache ("" = none)
     std::string include_dir; // device library headers for hiprtc
-    int waves_per_eu = 6;    // occupancy target of emitted kernels (0: compiler default)
+    int waves_per_eu = -1;   // occupancy target of emitted kernels (0: compiler default, -1: by kernel)
     bool closure_sample = false;  // emit CompositeBSDF::sample into surface kernels
     bool closure_export = false;  // emit the closure export into surface kernels
     mutable XformTable xf;

@@ -1,4 +1,5 @@
-"""Liveness of noise results in the emitter (no GPU needed)."""
+"""Emitter rules that choose what a kernel holds and its occupancy target (no
+GPU needed)."""
 import os
 
 from openshadinglanguage_amd import groupgen as G
@@ -44,3 +45,17 @@ def test_unread_gabor_is_left_out():
         gg = S.build_generated_group(ss, ([("cond_" + op, "surface", o.text())], []),
                                      "cond_" + op, outputs=["F"])
         assert "gabor(gu_" in ss.emit(gg)
+
+
+def test_occupancy_target_by_kernel():
+    """Unset, the target follows the kernel's closures; a set one holds."""
+    for mode, want in ((None, 3), ("closure_sample", 3), ("closure_export", 2)):
+        ss = S.ShadingSystem()
+        if mode:
+            ss.attribute(mode, 1)
+        ss, g = S.build_mx_layered(ss)
+        assert "amdgpu_waves_per_eu(%d)" % want in ss.emit(g), mode
+        ss.attribute("gpu_waves_per_eu", 5)
+        assert "amdgpu_waves_per_eu(5)" in ss.emit(g)
+    ss, g = S.build_layered3()
+    assert "amdgpu_waves_per_eu(6)" in ss.emit(g)
