@@ -26,7 +26,7 @@ HIPFLAGS = [
 
 # Per-source extra flags. The surrogate's MFMA kernels keep their
 # accumulators in VGPRs (the SiLU reads them there) instead of the
-# accumulation registers, which then hold the inference weights.
+# accumulation registers.
 EXTRA_FLAGS = {"oslmi_surrogate.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 

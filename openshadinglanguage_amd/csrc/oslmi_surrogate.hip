@@ -16,13 +16,12 @@
 // weights and refreshes the packed bf16 copies. No atomics: training is
 // deterministic.
 //
-// Inference: one fused kernel. Each wave keeps every weight fragment in the
-// accumulation registers (the MFMA reads its A operand there), reads the
-// bias initialisers from LDS, and walks pairs of 16-query column tiles: a
-// layer's MFMA accumulators (lane: 4 consecutive features of one query, in
-// VGPRs) become the next layer's B operand in place, because the packed
+// Inference: one fused kernel. Every weight fragment sits in LDS, shared by
+// the waves of a workgroup, and each wave walks pairs of 16-query column
+// tiles: a layer's MFMA accumulators (lane: 4 consecutive features of one
+// query) become the next layer's B operand in place, because the packed
 // weight fragments use the matching order of the 64 hidden features along
-// K. That fits a wave in 240 registers, two waves per SIMD. The SiLU costs
+// K. That fits a wave in 128 registers, four waves per SIMD. The SiLU costs
 // two transcendentals (exp2, rcp) and two VALU operations per unit, with
 // the -log2(e) scaling folded into the packed weights, and the output
 // epilogue is one exp2 (output normalisation folded into W5 and b5).
@@ -385,7 +384,7 @@ __global__ __launch_bounds__(256) void k_reduce_adam(const float* __restrict__ p
 // ---- inference ---------------------------------------------------------
 // Packed fragments: 30 per lane (W1 4 tiles; W2..W4 4 tiles x 2 K steps;
 // W5 1 tile x 2 K steps), 8 bf16 each, stored [fragment][lane]; biases as
-// accumulator initialisers: 17 float4 per lane, stored [slot][lane].
+// accumulator initialisers: 17 float4 per lane group, stored [slot][group].
 constexpr int NFRAG = 30, NBIAS = 17;
 constexpr int NCELL = 64;
 
@@ -437,16 +436,16 @@ __device__ __forceinline__ int route_cell(float lx, float lz, float vx, float vz
 }
 
 // Class of a query: 0 exact zero (V.z > 0 and L.z <= 0), 1 network
-// (inside the training domain and, in mode 1, not in a routed cell), 2
-// fallback (mode 1: the exact closure) or unanswered (mode 0: NaN).
-__device__ __forceinline__ int route_class(const Domain& dom, unsigned long long cell_mask, int mode,
+// (inside the training domain in[5..13] and, in mode 1, not in a routed
+// cell), 2 fallback (mode 1: the exact closure) or unanswered (mode 0: NaN).
+__device__ __forceinline__ int route_class(const f32x4 in[NIN], unsigned long long cell_mask, int mode,
                                            const float v[NIN])
 {
     const float lz = v[2], vz = v[4];
     bool inside = vz > 0.0f;
 #pragma unroll
-    for (int k = 0; k < 9; k++)
-        inside = inside && v[5 + k] >= dom.lo[k] && v[5 + k] <= dom.hi[k];
+    for (int k = 5; k < NIN; k++)
+        inside = inside && v[k] >= in[k][2] && v[k] <= in[k][3];
     const int cell = route_cell(v[0], lz, v[3], vz, v[6]);
     if (inside && mode == 1 && ((cell_mask >> cell) & 1ull))
         inside = false;
@@ -455,110 +454,94 @@ __device__ __forceinline__ int route_class(const Domain& dom, unsigned long long
     return inside ? 1 : 2;
 }
 
-// Per-wave queue of network queries in LDS: a ring of QCAP slots of 16
-// floats (14 raw inputs, the query index as bits, padding).
-constexpr int QCAP = 96, QSLOT = 16, WAVES_PER_BLOCK = 4;
-static_assert(QSLOT == 16, "slot reads index with k & (QSLOT - 1)");
+// Per-wave queue of network queries in LDS: a ring of QCAP slots in two
+// arrays of 16 bytes a slot (the layer-1 operand of a lane group each):
+// inputs 0..7, then inputs 8..13 and the query index; inputs normalised and
+// rounded to bf16 when queued. Rounds of 32 queries never wrap (QCAP is a
+// multiple of 32).
+constexpr int QCAP = 96, WAVES_PER_BLOCK = 8;
+static_assert(QCAP % 32 == 0 && QCAP >= 32 + 64 - 1, "a chunk of 64 joins up to 31 pending queries");
 // Per-wave fallback list in LDS (flushed to the global list when full).
 constexpr int FBCAP = 64;
 
-// The network over TILES 16-query tiles whose inputs sit in queue slots
-// head + 16 u + r (u < TILES, r = lane % 16) of this wave's ring; `count`
-// of them are valid. Writes the outputs (or appends to the fallback list).
-template<int TILES>
-__device__ __forceinline__ void run_tiles(const float* __restrict__ ring, int head, int count,
-                                          const float noff[8], const float nscl[8],
-                                          const bf16x8 w1[4], const bf16x8 w2[4][2],
-                                          const bf16x8 w3[4][2], const bf16x8 w4[4][2],
-                                          const bf16x8 w5[2], const f32x4* __restrict__ s_b,
-                                          int64_t n, float* __restrict__ out, bool spot_check,
-                                          float min_weight, bool spot[TILES], int qi_out[TILES])
+struct InferLds {
+    bf16x8 w[NFRAG * 64];   // weight fragments [fragment][lane]
+    f32x4 b[NBIAS * 4];     // accumulator initialisers [slot][lane / 16]
+    uint4 lo[WAVES_PER_BLOCK][QCAP], hi[WAVES_PER_BLOCK][QCAP];
+    int fb[WAVES_PER_BLOCK][FBCAP];
+    // per input: normalisation offset and scale, domain bounds (kept here:
+    // 46 uniform values more than the scalar registers hold)
+    f32x4 in[NIN];
+};
+
+// The network over two 16-query tiles whose inputs sit in slots head + 16 u
+// + r (r = lane % 16) of this wave's ring; `count` of them are valid. Writes
+// the outputs, or flags queries for the exact closure (spot, qi_out).
+__device__ __forceinline__ void run_tiles(const InferLds& L, int wv, int head, int count, int64_t n,
+                                          float* __restrict__ out, bool spot_check,
+                                          float min_weight, bool spot[2], int qi_out[2])
 {
+    // the fragments are read again each time: kept over the loop they would
+    // take 120 registers, and with them half of the waves
+    asm volatile("" ::: "memory");
     const int lane = threadIdx.x & 63;
     const int g = lane >> 4, r = lane & 15;
-    bf16x8 x[TILES];
-    int qi[TILES];
+    auto w = [&](int f) { return L.w[f * 64 + lane]; };
+    auto bias = [&](int f) { return L.b[f * 4 + g]; };
+    bf16x8 x[2];
+    int qi[2];
+    const uint32_t m = g < 2 ? ~0u : 0u, m3 = g == 0 ? ~0u : 0u;
 #pragma unroll
-    for (int u = 0; u < TILES; u++) {
-        const int e     = u * 16 + r;
-        const float* sl = ring + ((head + e) % QCAP) * QSLOT;
-        // the whole slot is read unconditionally (always inside the ring)
-        // and masked afterwards: conditional reads made the compiler wait
-        // for every outstanding global load, the next chunk's included
-        const int qv = __float_as_int(sl[14]);
-        qi[u]        = e < count ? qv : -1;
+    for (int u = 0; u < 2; u++) {
+        const int e = head + 16 * u + r;
+        uint4 v     = g == 1 ? L.hi[wv][e] : L.lo[wv][e];
+        v.x &= m;  // lane groups 2 and 3 hold the padding inputs 16..31,
+        v.y &= m;  // the last word of group 1 the query index
+        v.z &= m;
+        v.w &= m3;
+        x[u]  = __builtin_bit_cast(bf16x8, v);
+        qi[u] = 16 * u + r < count ? (int)L.hi[wv][e].w : -1;
+    }
+    f32x4 a[2][4];
+    bf16x8 h0[2], h1[2];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            // layer-1 operand: this lane group's 8 inputs (normalised)
-            const int k   = 8 * g + j;
-            const float v = sl[k & (QSLOT - 1)];  // inside the slot; k >= NIN masked
-            x[u][j] = (bf16)(k < NIN && e < count ? (v - noff[j]) * nscl[j] : 0.0f);
+    for (int t = 0; t < 4; t++) {
+        const bf16x8 wt = w(t);
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+            a[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt, x[u], bias(t), 0, 0, 0);
+    }
+#pragma unroll
+    for (int l = 0; l < 3; l++) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            h0[u] = act_pair(a[u][0], a[u][1]);
+            h1[u] = act_pair(a[u][2], a[u][3]);
         }
-    }
-    f32x4 a[TILES][4];
-    bf16x8 h0[TILES], h1[TILES];
-    f32x4 y2[TILES];
-#pragma unroll
-    for (int u = 0; u < TILES; u++)
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-            a[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1[t], x[u], s_b[t * 64 + lane], 0, 0, 0);
-#pragma unroll
-    for (int u = 0; u < TILES; u++) {
-        h0[u] = act_pair(a[u][0], a[u][1]);
-        h1[u] = act_pair(a[u][2], a[u][3]);
-    }
-#pragma unroll
-    for (int u = 0; u < TILES; u++)
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-            a[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w2[t][0], h0[u], s_b[(4 + t) * 64 + lane], 0, 0, 0);
-            a[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w2[t][1], h1[u], a[u][t], 0, 0, 0);
+            const bf16x8 w0 = w(4 + 8 * l + 2 * t), w1 = w(4 + 8 * l + 2 * t + 1);
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                a[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0, h0[u], bias(4 + 4 * l + t), 0, 0, 0);
+                a[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, h1[u], a[u][t], 0, 0, 0);
+            }
         }
-#pragma unroll
-    for (int u = 0; u < TILES; u++) {
-        h0[u] = act_pair(a[u][0], a[u][1]);
-        h1[u] = act_pair(a[u][2], a[u][3]);
-    }
-#pragma unroll
-    for (int u = 0; u < TILES; u++)
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            a[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w3[t][0], h0[u], s_b[(8 + t) * 64 + lane], 0, 0, 0);
-            a[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w3[t][1], h1[u], a[u][t], 0, 0, 0);
-        }
-#pragma unroll
-    for (int u = 0; u < TILES; u++) {
-        h0[u] = act_pair(a[u][0], a[u][1]);
-        h1[u] = act_pair(a[u][2], a[u][3]);
-    }
-#pragma unroll
-    for (int u = 0; u < TILES; u++)
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            a[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w4[t][0], h0[u], s_b[(12 + t) * 64 + lane], 0, 0, 0);
-            a[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w4[t][1], h1[u], a[u][t], 0, 0, 0);
-        }
-#pragma unroll
-    for (int u = 0; u < TILES; u++) {
-        h0[u] = act_pair(a[u][0], a[u][1]);
-        h1[u] = act_pair(a[u][2], a[u][3]);
-    }
-#pragma unroll
-    for (int u = 0; u < TILES; u++) {
-        y2[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w5[0], h0[u], s_b[16 * 64 + lane], 0, 0, 0);
-        y2[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w5[1], h1[u], y2[u], 0, 0, 0);
     }
     // lanes of group 0 hold outputs 0..3 of their query. Spot check (when
     // spot_check): a predicted weight below the threshold has a large
     // relative error (the log-space fit is absolute); such a query is not
     // written but flagged in spot[u] / qi_out[u] for the exact closure.
 #pragma unroll
-    for (int u = 0; u < TILES; u++) {
+    for (int u = 0; u < 2; u++) {
+        h0[u]   = act_pair(a[u][0], a[u][1]);
+        h1[u]   = act_pair(a[u][2], a[u][3]);
+        f32x4 y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w(28), h0[u], bias(16), 0, 0, 0);
+        y       = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w(29), h1[u], y, 0, 0, 0);
         float v[4];
 #pragma unroll
         for (int o = 0; o < 4; o++)
-            v[o] = __builtin_amdgcn_exp2f(y2[u][o]);
+            v[o] = __builtin_amdgcn_exp2f(y[o]);
         const bool mine = g == 0 && qi[u] >= 0;
         spot[u]   = spot_check && mine && fminf(fminf(v[0], v[1]), v[2]) < min_weight;
         qi_out[u] = qi[u];
@@ -578,26 +561,30 @@ __device__ __forceinline__ void run_tiles(const float* __restrict__ ring, int he
 // compaction, query order kept). Whenever 32 are queued, the network runs
 // on two 16-query tiles; the rest is flushed after the last chunk. The next
 // chunk's inputs are loaded before the network runs on the current queue.
-// The weights stay in the accumulation registers for the whole kernel (the
-// MFMA reads its A operand there), the bias initialisers in LDS.
-template<int TILES>
-__global__ __launch_bounds__(256) void k_infer_fused(InferConsts kc, unsigned long long cell_mask,
-                                                     int mode, const bf16x8* __restrict__ frag,
-                                                     const f32x4* __restrict__ biasp,
-                                                     const float* __restrict__ q, int64_t n,
-                                                     float* __restrict__ out, float min_weight,
-                                                     int* __restrict__ fbidx, int* __restrict__ fbcount)
+// What bounds it is the SiLU: of the about 4200 issue cycles that 32 queries
+// take, 256 exp2 and rcp take 2900. Measured over 8M queries, 4.19M of them
+// for the network (with the exact fallback): 350 us; 412 with the weights in
+// the accumulation registers, the ring in fp32 and two waves per SIMD; 397
+// with five waves (ten to a workgroup: two SIMDs carry more); 353 with
+// 8-byte loads of two queries a lane.
+__global__ __launch_bounds__(64 * WAVES_PER_BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void k_infer_fused(InferConsts kc, unsigned long long cell_mask, int mode,
+                   const bf16x8* __restrict__ frag, const f32x4* __restrict__ biasp,
+                   const float* __restrict__ q, int64_t n, float* __restrict__ out,
+                   float min_weight, int* __restrict__ fbidx, int* __restrict__ fbcount)
 {
-    __shared__ f32x4 s_b[NBIAS * 64];
-    __shared__ float s_ring[WAVES_PER_BLOCK][QCAP * QSLOT];
-    __shared__ int s_fb[WAVES_PER_BLOCK][FBCAP];
-    for (int j = threadIdx.x; j < NBIAS * 64; j += blockDim.x)
-        s_b[j] = biasp[j];
+    __shared__ InferLds L;
+    for (int j = threadIdx.x; j < NFRAG * 64; j += blockDim.x)
+        L.w[j] = frag[j];
+    if (threadIdx.x < NBIAS * 4)
+        L.b[threadIdx.x] = biasp[threadIdx.x];
+    if (threadIdx.x < NIN) {
+        const int k     = threadIdx.x, d = k < 5 ? 0 : k - 5;
+        L.in[k] = f32x4 { kc.nm.in_off[k], kc.nm.in_scale[k], kc.dom.lo[d], kc.dom.hi[d] };
+    }
     __syncthreads();
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int g    = lane >> 4;
-    float* ring    = s_ring[wv];
-    int* fbl       = s_fb[wv];
+    int* fbl       = L.fb[wv];
     const unsigned long long lt = (1ull << lane) - 1ull;
     // this wave's fallback list: fbn (wave-uniform) indices in fbl, moved
     // to the global list with one atomic when full and at the end
@@ -626,39 +613,6 @@ __global__ __launch_bounds__(256) void k_infer_fused(InferConsts kc, unsigned lo
         fbn += cnt;
         __builtin_amdgcn_wave_barrier();
     };
-    bf16x8 w1[4], w2[4][2], w3[4][2], w4[4][2], w5[2];
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        w1[t] = frag[t * 64 + lane];
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            w2[t][s] = frag[(4 + t * 2 + s) * 64 + lane];
-            w3[t][s] = frag[(12 + t * 2 + s) * 64 + lane];
-            w4[t][s] = frag[(20 + t * 2 + s) * 64 + lane];
-        }
-    }
-    w5[0] = frag[28 * 64 + lane];
-    w5[1] = frag[29 * 64 + lane];
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        asm volatile("" : "+a"(w1[t]));
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            asm volatile("" : "+a"(w2[t][s]));
-            asm volatile("" : "+a"(w3[t][s]));
-            asm volatile("" : "+a"(w4[t][s]));
-        }
-    }
-    asm volatile("" : "+a"(w5[0]));
-    asm volatile("" : "+a"(w5[1]));
-    // this lane group's normalisation constants (inputs 8g .. 8g+7)
-    float noff[8], nscl[8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int k = 8 * g + j;
-        noff[j]     = k < NIN ? kc.nm.in_off[k < NIN ? k : 0] : 0.0f;
-        nscl[j]     = k < NIN ? kc.nm.in_scale[k < NIN ? k : 0] : 0.0f;
-    }
     const int64_t nchunks = (n + 63) / 64;
     const int64_t wave    = (int64_t)blockIdx.x * WAVES_PER_BLOCK + wv;
     const int64_t nwaves  = (int64_t)gridDim.x * WAVES_PER_BLOCK;
@@ -677,7 +631,7 @@ __global__ __launch_bounds__(256) void k_infer_fused(InferConsts kc, unsigned lo
     for (int64_t chunk = wave; chunk < nchunks; chunk += nwaves) {
         const int64_t i = chunk * 64 + lane;
         const bool live = i < n;
-        int c = live ? route_class(kc.dom, cell_mask, mode, cur) : -1;
+        int c = live ? route_class(L.in, cell_mask, mode, cur) : -1;
         if (c == 0) {
             out[i] = out[n + i] = out[2 * n + i] = out[3 * n + i] = 0.0f;
         } else if (c == 2 && mode == 0) {
@@ -687,40 +641,42 @@ __global__ __launch_bounds__(256) void k_infer_fused(InferConsts kc, unsigned lo
             fb_append(c == 2, (int)i);
         const unsigned long long nb = __ballot(c == 1);
         if (c == 1) {
-            float* sl = ring + ((head + pending + __popcll(nb & lt)) % QCAP) * QSLOT;
+            bf16x8 lo, hi;
 #pragma unroll
-            for (int k = 0; k < NIN; k++)
-                sl[k] = cur[k];
-            sl[14] = __int_as_float((int)i);
+            for (int k = 0; k < NIN; k++) {
+                const bf16 v = (bf16)((cur[k] - L.in[k][0]) * L.in[k][1]);
+                if (k < 8)
+                    lo[k] = v;
+                else
+                    hi[k - 8] = v;
+            }
+            hi[6] = hi[7] = (bf16)0.0f;
+            uint4 hv = __builtin_bit_cast(uint4, hi);
+            hv.w     = (uint32_t)i;
+            int slot = head + pending + __popcll(nb & lt);
+            slot     = slot >= QCAP ? slot - QCAP : slot;
+            L.lo[wv][slot] = __builtin_bit_cast(uint4, lo);
+            L.hi[wv][slot] = hv;
         }
         pending += __popcll(nb);
         __builtin_amdgcn_wave_barrier();
         // the next chunk's inputs are in flight while the network runs
         if (chunk + nwaves < nchunks)
             load(chunk + nwaves, cur);
-        while (pending >= 16 * TILES) {
-            bool spot[TILES];
-            int qs[TILES];
-            run_tiles<TILES>(ring, head, 16 * TILES, noff, nscl, w1, w2, w3, w4, w5, s_b, n, out,
-                             mode == 1, min_weight, spot, qs);
-            head = (head + 16 * TILES) % QCAP;
-            pending -= 16 * TILES;
+        const bool end = chunk + nwaves >= nchunks;
+        while (pending >= 32 || (end && pending > 0)) {
+            const int count = pending < 32 ? pending : 32;
+            bool spot[2];
+            int qs[2];
+            run_tiles(L, wv, head, count, n, out, mode == 1, min_weight, spot, qs);
+            head = head + 32 == QCAP ? 0 : head + 32;
+            pending -= count;
             __builtin_amdgcn_wave_barrier();
             if (mode == 1)
 #pragma unroll
-                for (int u = 0; u < TILES; u++)
+                for (int u = 0; u < 2; u++)
                     fb_append(spot[u], qs[u]);
         }
-    }
-    if (pending > 0) {
-        bool spot[TILES];
-        int qs[TILES];
-        run_tiles<TILES>(ring, head, pending, noff, nscl, w1, w2, w3, w4, w5, s_b, n, out,
-                         mode == 1, min_weight, spot, qs);
-        if (mode == 1)
-#pragma unroll
-            for (int u = 0; u < TILES; u++)
-                fb_append(spot[u], qs[u]);
     }
     if (mode == 1)
         fb_flush();
@@ -760,7 +716,7 @@ int ctx_alloc(Context* c)
         { (void**)&c->P, NPARAM * 4 }, { (void**)&c->Mm, NPARAM * 4 }, { (void**)&c->Vv, NPARAM * 4 },
         { (void**)&c->G, NPARAM * 4 }, { (void**)&c->fwd, NFWD * 64 * 16 }, { (void**)&c->bwd, NBWD * 64 * 16 },
         { (void**)&c->part, (size_t)nb * NPARAM * 4 }, { (void**)&c->lpart, (size_t)nb * 4 },
-        { (void**)&c->frag, (size_t)NFRAG * 64 * 16 }, { (void**)&c->biasp, (size_t)NBIAS * 64 * 16 },
+        { (void**)&c->frag, (size_t)NFRAG * 64 * 16 }, { (void**)&c->biasp, (size_t)NBIAS * 4 * 16 },
     };
     for (auto& it : items) {
         if (int rc = check_hip(hipMalloc(it.p, it.bytes), "hipMalloc(surrogate)"))
@@ -809,7 +765,7 @@ int pack_inference(Context* c)
 {
     const std::vector<float>& P = c->host_params;
     std::vector<bf16> frag((size_t)NFRAG * 64 * 8);
-    std::vector<float> bias((size_t)NBIAS * 64 * 4);
+    std::vector<float> bias((size_t)NBIAS * 4 * 4);
     auto W = [&](int l, int o, int i) { return P[OFF_W[l] + o * LAYER_IN[l] + i]; };
     int f = 0;
     for (int t = 0; t < 4; t++, f++)
@@ -832,17 +788,16 @@ int pack_inference(Context* c)
     int b = 0;
     for (int l = 1; l <= 4; l++)
         for (int t = 0; t < 4; t++, b++)
-            for (int lane = 0; lane < 64; lane++)
+            for (int g = 0; g < 4; g++)
                 for (int j = 0; j < 4; j++)
-                    bias[((size_t)b * 64 + lane) * 4 + j] =
-                        -kLog2e * P[OFF_B[l] + 16 * t + 4 * (lane >> 4) + j];
-    for (int lane = 0; lane < 64; lane++)
+                    bias[((size_t)b * 4 + g) * 4 + j] = -kLog2e * P[OFF_B[l] + 16 * t + 4 * g + j];
+    for (int g = 0; g < 4; g++)
         for (int j = 0; j < 4; j++) {
-            const int o = 4 * (lane >> 4) + j;
+            const int o = 4 * g + j;
             float v     = P[OFF_B[5] + o];
             if (o < NOUT)
                 v = (v * c->nm.out_sd[o] + c->nm.out_mu[o]) * kLog2e;
-            bias[((size_t)b * 64 + lane) * 4 + j] = v;
+            bias[((size_t)b * 4 + g) * 4 + j] = v;
         }
     if (int rc = check_hip(hipMemcpy(c->frag, frag.data(), frag.size() * sizeof(bf16),
                                      hipMemcpyHostToDevice), "hipMemcpy(fragments)"))
@@ -1050,8 +1005,8 @@ extern "C" int oslmi_surrogate_set_spot_check(oslmi_surrogate* s, float min_weig
 }
 
 // Persistent grid of the fused kernel: the workgroups that fit at once (two
-// waves per SIMD: 228 of the 512 registers per lane, so 2 workgroups of 4
-// waves per CU), fewer when there are fewer 64-query chunks than waves.
+// of eight waves per CU: 128 registers, 58 KB of LDS), fewer when there are
+// fewer 64-query chunks than waves.
 static unsigned infer_grid(int64_t n)
 {
     const int64_t chunks = (n + 63) / 64;
@@ -1082,7 +1037,7 @@ extern "C" int oslmi_surrogate_infer(oslmi_surrogate* s, const oslmi_layered_mat
         return set_error(OSLMI_ERR_INVALID, "oslmi_surrogate_infer: fallback buffers needed");
     if (mode == 1)
         hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, st, d_fallback_count);
-    hipLaunchKernelGGL(k_infer_fused<2>, dim3(infer_grid(n)), dim3(256), 0, st, kc, s->c.cell_mask, mode,
+    hipLaunchKernelGGL(k_infer_fused, dim3(infer_grid(n)), dim3(64 * WAVES_PER_BLOCK), 0, st, kc, s->c.cell_mask, mode,
                        s->c.frag, s->c.biasp, d_query, n, d_out, s->c.min_weight,
                        mode == 1 ? d_fallback_index : nullptr,
                        mode == 1 ? d_fallback_count : nullptr);
