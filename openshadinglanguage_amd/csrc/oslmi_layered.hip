@@ -162,7 +162,7 @@ void bake_tables(float* out)
             auto w          = [&](V3 wo, V3 rnd) {
                 if (wo.z <= 0)
                     return 0.0f;
-                const V3 m  = ggx_sample_bvndf<TrigLibm>(sp.d, wo, rnd.x, rnd.y);
+                const V3 m  = ggx_sample_bvndf<TrigLibm>(sp.d, ggx_bvndf_terms(sp.d, wo), rnd.x, rnd.y);
                 const V3 wi = reflect(wo, m);
                 if (wi.z <= 0)
                     return 0.0f;
@@ -280,9 +280,11 @@ struct Layered {
     float s_a, s_Emiss;
     MicroLobe coat, base;
     WoTerms coat_t, base_t;
+    BvndfTerms coat_b, base_b;  // layered_sample_terms
     int n;  // lobes present: sheen, then coat, then base
     V3 w[3];
     float pdf[3];
+    float inv_pdf[3];  // 1 / pdf
 };
 
 // SheenLobe::eval_impl (front facing)
@@ -420,31 +422,40 @@ OSLMI_DEV void layered_build(Layered* L, const Material& mat, V3 N, V3 wo, float
             if (i < L->n)
                 L->pdf[i] = L->pdf[i] / total;
     }
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+        L->inv_pdf[i] = 1 / L->pdf[i];
 }
 
-OSLMI_DEV void mis_update(V3* w, float* pdf, V3 ow, float opdf, float b)
+// What the four samples of a point share
+template<bool SAME> OSLMI_DEV void layered_sample_terms(Layered* L)
+{
+    L->coat_b = ggx_bvndf_terms(L->coat.sp.d, L->wo_m);
+    if (!SAME)
+        L->base_b = ggx_bvndf_terms(L->base.sp.d, L->wo_m);
+}
+
+// MIS::update_eval; inv_b = 1 / b. Both of its cases divide the smaller pdf
+// by the larger and take 1 / (1 + the quotient).
+OSLMI_DEV void mis_update(V3* w, float* pdf, V3 ow, float opdf, float b, float inv_b)
 {
     if (b > kFLT_MIN) {
         opdf *= b;
-        ow = ow * (1 / b);
-        float mis;
-        if (*pdf < opdf)
-            mis = 1 / (1 + *pdf / opdf);
-        else if (opdf < *pdf)
-            mis = 1 - 1 / (1 + opdf / *pdf);
-        else
-            mis = 0.5f;
+        ow              = ow * inv_b;
+        const bool less = *pdf < opdf;
+        const float t   = 1 / (1 + (less ? *pdf : opdf) / (less ? opdf : *pdf));
+        const float mis = less ? t : (opdf < *pdf ? 1 - t : 0.5f);
         *w = *w * (1 - mis) + ow * mis;
         *pdf += opdf;
     }
 }
 // mis_update of a zero weight and pdf (the sheen, evaluated first): its two
 // quotients are 0 and 1
-OSLMI_DEV void mis_first(V3* w, float* pdf, V3 ow, float opdf, float b)
+OSLMI_DEV void mis_first(V3* w, float* pdf, V3 ow, float opdf, float b, float inv_b)
 {
     if (b > kFLT_MIN) {
         opdf *= b;
-        ow              = ow * (1 / b);
+        ow              = ow * inv_b;
         const float mis = 0.0f < opdf ? 1.0f : 0.5f;
         *w              = V3(0.0f) + ow * mis;
         *pdf            = opdf;
@@ -459,14 +470,14 @@ template<bool SAME> OSLMI_DEV void layered_eval(const Layered& L, V3 wi, V3* wei
     const V3 wi_s = L.fs.local(wi);
     const V3 wi_m = L.fm.local(wi);
     Sample b      = sheen_eval(L, L.wo_s, wi_s);
-    mis_first(&sw, &sp, b.weight * L.w[0], b.pdf, L.pdf[0]);
+    mis_first(&sw, &sp, b.weight * L.w[0], b.pdf, L.pdf[0], L.inv_pdf[0]);
     if (L.n > 1) {
         const Refl g = turquin_geometry(L.coat.sp.d, L.coat_t, L.wo_m, wi_m);
         b            = micro_eval(L.coat, g);
-        mis_update(&sw, &sp, b.weight * L.w[1], b.pdf, L.pdf[1]);
+        mis_update(&sw, &sp, b.weight * L.w[1], b.pdf, L.pdf[1], L.inv_pdf[1]);
         if (L.n > 2) {
             b = micro_eval(L.base, SAME ? g : turquin_geometry(L.base.sp.d, L.base_t, L.wo_m, wi_m));
-            mis_update(&sw, &sp, b.weight * L.w[2], b.pdf, L.pdf[2]);
+            mis_update(&sw, &sp, b.weight * L.w[2], b.pdf, L.pdf[2], L.inv_pdf[2]);
         }
     }
     *weight = sw;
@@ -477,6 +488,7 @@ template<bool SAME> OSLMI_DEV void layered_eval(const Layered& L, V3 wi, V3* wei
 // direction in its frame; every present lobe is then evaluated at it (the
 // chosen one at its local direction, as the lobe's own sample does) and
 // the others are MIS-combined in closure order.
+template<bool SAME>
 OSLMI_DEV void layered_sample(const Layered& L, float rx, float ry, V3* wi_out, V3* weight,
                               float* pdf)
 {
@@ -484,14 +496,13 @@ OSLMI_DEV void layered_sample(const Layered& L, float rx, float ry, V3* wi_out, 
     *weight  = V3(0.0f);
     *pdf     = 0.0f;
     int pick = -1;
-    float accum = 0;
+    float accum = 0, pick_pdf = 0;
 #pragma unroll
     for (int i = 0; i < 3; i++) {
         if (pick < 0 && i < L.n) {
             if (rx < (L.pdf[i] + accum)) {
-                pick = i;
-                rx   = (rx - accum) / L.pdf[i];
-                rx   = smin(rx, 0.99999994f);
+                pick     = i;
+                pick_pdf = L.pdf[i];
             } else {
                 accum += L.pdf[i];
             }
@@ -499,14 +510,16 @@ OSLMI_DEV void layered_sample(const Layered& L, float rx, float ry, V3* wi_out, 
     }
     if (pick < 0)
         return;
+    rx = (rx - accum) / pick_pdf;
+    rx = smin(rx, 0.99999994f);
     V3 wl;
     if (pick == 0) {
         wl = sample_uniform_hemisphere(rx, ry);
     } else {
-        const MicroLobe& M = pick == 1 ? L.coat : L.base;
-        if (!M.dorefl || L.wo_m.z <= 0)
+        if (!(pick == 1 ? L.coat.dorefl : L.base.dorefl) || L.wo_m.z <= 0)
             return;
-        const V3 m = ggx_sample_bvndf<TrigFast>(M.sp.d, L.wo_m, rx, ry);
+        const V3 m = SAME || pick == 1 ? ggx_sample_bvndf<TrigFast>(L.coat.sp.d, L.coat_b, rx, ry)
+                                       : ggx_sample_bvndf<TrigFast>(L.base.sp.d, L.base_b, rx, ry);
         wl         = reflect(L.wo_m, m);
         if (wl.z <= 0 || MAX_ABS_XYZ(wl) < kEPSILON)
             return;
@@ -527,7 +540,7 @@ OSLMI_DEV void layered_sample(const Layered& L, float rx, float ry, V3* wi_out, 
 #pragma unroll
     for (int j = 0; j < 3; j++) {
         if (j == pick) {
-            sw = b[j].weight * (L.w[j] * (1 / L.pdf[j]));
+            sw = b[j].weight * (L.w[j] * L.inv_pdf[j]);
             sp = b[j].pdf * L.pdf[j];
         }
     }
@@ -536,7 +549,7 @@ OSLMI_DEV void layered_sample(const Layered& L, float rx, float ry, V3* wi_out, 
 #pragma unroll
     for (int j = 0; j < 3; j++)
         if (j < L.n && j != pick)
-            mis_update(&sw, &sp, b[j].weight * L.w[j], b[j].pdf, L.pdf[j]);
+            mis_update(&sw, &sp, b[j].weight * L.w[j], b[j].pdf, L.pdf[j], L.inv_pdf[j]);
     *wi_out = wi;
     *weight = sw;
     *pdf    = sp;
@@ -545,7 +558,7 @@ OSLMI_DEV void layered_sample(const Layered& L, float rx, float ry, V3* wi_out, 
 // ---- kernels ---------------------------------------------------------------
 // Tables staged in LDS: 8448 floats (33 KB) per workgroup.
 template<bool SAME>
-__global__ __launch_bounds__(kLayeredBlock) void k_layered(Material mat, const float* __restrict__ lut,
+__global__ __launch_bounds__(kLayeredBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_layered(Material mat, const float* __restrict__ lut,
                                                  const float* __restrict__ Np,
                                                  const float* __restrict__ Vp,
                                                  const float* __restrict__ Lp,
@@ -576,11 +589,12 @@ __global__ __launch_bounds__(kLayeredBlock) void k_layered(Material mat, const f
             eval[3 * n + i] = p;
         }
         if (samp) {
+            layered_sample_terms<SAME>(&L);
 #pragma unroll 1
             for (int k = 0; k < 4; k++) {
                 V3 wi, w;
                 float p;
-                layered_sample(L, rnd[(2 * k) * n + i], rnd[(2 * k + 1) * n + i], &wi, &w, &p);
+                layered_sample<SAME>(L, rnd[(2 * k) * n + i], rnd[(2 * k + 1) * n + i], &wi, &w, &p);
                 float* o     = samp + (int64_t)(7 * k) * n;
                 o[i]         = wi.x;
                 o[n + i]     = wi.y;

@@ -275,24 +275,35 @@ OSLMI_HD V3 ggx_sample_vndf(const GGX& d, V3 wo, float randu, float randv)
     const V3 N      = px * T1 + p2o * T2 + p3 * V;
     return normalized(V3(d.ax * N.x, d.ay * N.y, smax(N.z, 0.0f)));
 }
-// bounded visible-normal sampling for reflection (Eto-Tokuyoshi); Trig::sc
-// gives sin and cos of the azimuth
-template<class Trig> OSLMI_HD V3 ggx_sample_bvndf(const GGX& d, V3 wo, float randu, float randv)
+// bounded visible-normal sampling for reflection (Eto-Tokuyoshi): what it
+// needs of wo alone, and the microfacet normal; Trig::sc gives sin and cos of
+// the azimuth
+struct BvndfTerms {
+    V3 i_std;
+    float b;
+};
+OSLMI_HD BvndfTerms ggx_bvndf_terms(const GGX& d, V3 wo)
 {
-    V3 i_std             = normalized(V3(wo.x * d.ax, wo.y * d.ay, wo.z));
+    BvndfTerms t;
+    t.i_std        = normalized(V3(wo.x * d.ax, wo.y * d.ay, wo.z));
+    const float a  = CLAMP(smin(d.ax, d.ay), 0.0f, 1.0f);
+    const float s  = 1 + sqrtf(SQR(wo.x) + SQR(wo.y));
+    const float a2 = SQR(a);
+    const float s2 = SQR(s);
+    const float k  = (1 - a2) * s2 / (s2 + a2 * SQR(wo.z));
+    t.b            = k * t.i_std.z;
+    return t;
+}
+template<class Trig>
+OSLMI_HD V3 ggx_sample_bvndf(const GGX& d, const BvndfTerms& t, float randu, float randv)
+{
     const float phi      = 2.0f * kPI * randu;
-    const float a        = CLAMP(smin(d.ax, d.ay), 0.0f, 1.0f);
-    const float s        = 1 + sqrtf(SQR(wo.x) + SQR(wo.y));
-    const float a2       = SQR(a);
-    const float s2       = SQR(s);
-    const float k        = (1 - a2) * s2 / (s2 + a2 * SQR(wo.z));
-    const float b        = k * i_std.z;
-    const float z        = (1 - randv) * (1 + b) - b;
+    const float z        = (1 - randv) * (1 + t.b) - t.b;
     const float sinTheta = sqrtf(CLAMP(1 - SQR(z), 0.0f, 1.0f));
     float sn, c;
     Trig::sc(phi, &sn, &c);
     V3 o_std = V3(sinTheta * c, sinTheta * sn, z);
-    V3 m_std = i_std + o_std;
+    V3 m_std = t.i_std + o_std;
     return normalized(V3(m_std.x * d.ax, m_std.y * d.ay, m_std.z));
 }
 struct TrigFast {
@@ -615,7 +626,7 @@ OSLMI_DEV bool mx_sample_dir(const MxLobe& M, int kind, float rx, float ry, V3* 
     }
     if (!M.dorefl || M.wol.z <= 0)
         return false;
-    const V3 m = ggx_sample_bvndf<TrigFast>(M.sp.d, M.wol, rx, ry);
+    const V3 m = ggx_sample_bvndf<TrigFast>(M.sp.d, ggx_bvndf_terms(M.sp.d, M.wol), rx, ry);
     *wl        = reflect(M.wol, m);
     return !(wl->z <= 0 || MAX_ABS_XYZ(*wl) < kEPSILON);
 }
