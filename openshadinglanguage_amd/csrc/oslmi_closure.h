@@ -445,13 +445,11 @@ OSLMI_DEV void mis_update(V3* w, float* pdf, V3 ow, float opdf, float b)
     if (b > 1.17549435e-38f) {
         opdf *= b;
         ow = ow * (1 / b);
-        float mis;
-        if (*pdf < opdf)
-            mis = 1 / (1 + *pdf / opdf);
-        else if (opdf < *pdf)
-            mis = 1 - 1 / (1 + opdf / *pdf);
-        else
-            mis = 0.5f;
+        // both cases divide the smaller pdf by the larger and take
+        // 1 / (1 + the quotient)
+        const bool less = *pdf < opdf;
+        const float t   = 1 / (1 + (less ? *pdf : opdf) / (less ? opdf : *pdf));
+        const float mis = less ? t : (opdf < *pdf ? 1 - t : 0.5f);
         *w = *w * (1 - mis) + ow * mis;
         *pdf += opdf;
     }
@@ -702,7 +700,10 @@ template<int MAXL> OSLMI_DEV BsdfEval composite_eval(const LobeList<MAXL>& L, V3
 
 // CompositeBSDF::sample: rx picks a lobe by the prepared pdfs and is
 // rescaled for it; the other lobes are evaluated at the drawn direction and
-// MIS-combined in closure order. Compile-time lobe slots throughout.
+// MIS-combined in closure order. Compile-time lobe slots throughout. The
+// picked lobe is selected into one variable first, so a wave whose lanes
+// picked different lobes runs one sample and one eval of each lobe; a
+// branch per pick ran every pick's sample and its evals of all others.
 template<int MAXL>
 OSLMI_DEV BsdfDirSample composite_sample(const LobeList<MAXL>& L, V3 wo, float rx, float ry,
                                          float rz)
@@ -711,36 +712,40 @@ OSLMI_DEV BsdfDirSample composite_sample(const LobeList<MAXL>& L, V3 wo, float r
     s.wi        = V3(0.0f);
     s.weight    = V3(0.0f);
     s.pdf       = 0.0f;
-    float accum = 0;
-    bool done   = false;
+    float accum = 0, pdf = 0;
+    int pick    = -1;
+    Lobe l      = L.l[0];
 #pragma unroll
     for (int i = 0; i < MAXL; i++) {
-        if (!done && i < L.n) {
+        if (pick < 0 && i < L.n) {
             if (rx < (L.pdf[i] + accum)) {
-                done    = true;
-                float u = (rx - accum) / L.pdf[i];
-                u       = fminf(u, 0.99999994f);
-                s       = lobe_sample(L.l[i], wo, u, ry, rz);
-                const V3 wsc = L.l[i].weight * (1 / L.pdf[i]);
-                s.weight     = s.weight * wsc;
-                s.pdf        = s.pdf * L.pdf[i];
-                if (s.pdf == 0.0f) {
-                    s.wi     = V3(0.0f);
-                    s.weight = V3(0.0f);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < MAXL; j++)
-                        if (j != i && j < L.n) {
-                            BsdfEval b = lobe_eval(L.l[j], wo, s.wi);
-                            mis_update(&s.weight, &s.pdf, b.weight * L.l[j].weight, b.pdf,
-                                       L.pdf[j]);
-                        }
-                }
+                pick = i;
+                pdf  = L.pdf[i];
+                l    = L.l[i];
             } else {
                 accum += L.pdf[i];
             }
         }
     }
+    if (pick < 0)
+        return s;
+    float u      = (rx - accum) / pdf;
+    u            = fminf(u, 0.99999994f);
+    s            = lobe_sample(l, wo, u, ry, rz);
+    const V3 wsc = l.weight * (1 / pdf);
+    s.weight     = s.weight * wsc;
+    s.pdf        = s.pdf * pdf;
+    if (s.pdf == 0.0f) {
+        s.wi     = V3(0.0f);
+        s.weight = V3(0.0f);
+        return s;
+    }
+#pragma unroll
+    for (int j = 0; j < MAXL; j++)
+        if (j != pick && j < L.n) {
+            BsdfEval b = lobe_eval(L.l[j], wo, s.wi);
+            mis_update(&s.weight, &s.pdf, b.weight * L.l[j].weight, b.pdf, L.pdf[j]);
+        }
     return s;
 }
 
