@@ -31,16 +31,21 @@ OSLMI_DEV void bjmix(uint32_t& a, uint32_t& b, uint32_t& c)
     c -= b;  c ^= rotl32(b, 4);  b += a;
 }
 
+// Seven steps x ^= y; x -= rotl32(y, k) over (c, b), (a, c), (b, a), (c, b),
+// (a, c), (b, a), (c, b). Complements are carried where they let a step run
+// as one rotation and one fused xor-add (v_xad_u32): ~((x ^ y) - r) is
+// (~x ^ y) + r, and with ny = ~y, (x ^ y) - rotl(y) is rotl(ny) - (x ^ ny).
+// 18 instructions instead of 21 (c comes from an addition or xor, into which
+// its complement folds); the hashes are half of a perlin or simplex noise.
 OSLMI_DEV uint32_t bjfinal(uint32_t a, uint32_t b, uint32_t c)
 {
-    c ^= b; c -= rotl32(b, 14);
-    a ^= c; a -= rotl32(c, 11);
-    b ^= a; b -= rotl32(a, 25);
-    c ^= b; c -= rotl32(b, 16);
-    a ^= c; a -= rotl32(c, 4);
-    b ^= a; b -= rotl32(a, 14);
-    c ^= b; c -= rotl32(b, 24);
-    return c;
+    const uint32_t nc = (~c ^ b) + rotl32(b, 14);
+    a                 = rotl32(nc, 11) - (a ^ nc);
+    uint32_t nb       = (~b ^ a) + rotl32(a, 25);
+    c                 = (nc ^ nb) + rotl32(nb, 16) + 1u;
+    a                 = (a ^ c) - rotl32(c, 4);
+    nb                = (nb ^ a) + rotl32(a, 14);
+    return rotl32(nb, 24) - (c ^ nb);
 }
 
 #define OSLMI_SEED(n) (0xdeadbeefu + ((uint32_t)(n) << 2) + 13u)
@@ -196,17 +201,30 @@ OSLMI_DEV Wrap make_wrap(float a, float b = 1.0f, float c = 1.0f, float d = 1.0f
 }
 
 // ----------------------------------------------------------------- perlin
+// sgn(h, bit): +1 or -1 by a bit of h. add_signed(su, u, sv, v): su u + sv v,
+// one rounding (the products with +-1 are exact), as negating and adding is.
+OSLMI_DEV float sgn(int h, int bit)
+{
+    return __uint_as_float(0x3f800000u | (((uint32_t)h << (31 - bit)) & 0x80000000u));
+}
 template<class T> struct NOps;
 template<> struct NOps<float> {
     static OSLMI_DEV float one() { return 1.0f; }
     static OSLMI_DEV float c(float x) { return x; }
-    static OSLMI_DEV float neg_if(float v, bool b) { return b ? -v : v; }
+    static OSLMI_DEV float add_signed(float su, float u, float sv, float v)
+    {
+        return __fmaf_rn(su, u, sv * v);
+    }
     static OSLMI_DEV float sel(bool b, float t, float f) { return b ? t : f; }
 };
 template<> struct NOps<Df> {
     static OSLMI_DEV Df one() { return Df(1.0f); }
     static OSLMI_DEV Df c(float x) { return Df(x); }
-    static OSLMI_DEV Df neg_if(const Df& v, bool b) { return b ? -v : v; }
+    static OSLMI_DEV Df add_signed(float su, const Df& u, float sv, const Df& v)
+    {
+        return Df(__fmaf_rn(su, u.v, sv * v.v), __fmaf_rn(su, u.dx, sv * v.dx),
+                  __fmaf_rn(su, u.dy, sv * v.dy));
+    }
     static OSLMI_DEV Df sel(bool b, const Df& t, const Df& f) { return b ? t : f; }
 };
 
@@ -256,14 +274,14 @@ template<class T> OSLMI_DEV T grad2(int hash, const T& x, const T& y)
     int h = hash & 7;
     T u   = NOps<T>::sel(h < 4, x, y);
     T v   = 2.0f * NOps<T>::sel(h < 4, y, x);
-    return NOps<T>::neg_if(u, h & 1) + NOps<T>::neg_if(v, h & 2);
+    return NOps<T>::add_signed(sgn(h, 0), u, sgn(h, 1), v);
 }
 template<class T> OSLMI_DEV T grad3(int hash, const T& x, const T& y, const T& z)
 {
     int h = hash & 15;
     T u   = NOps<T>::sel(h < 8, x, y);
     T v   = NOps<T>::sel(h < 4, y, NOps<T>::sel((h == 12) || (h == 14), x, z));
-    return NOps<T>::neg_if(u, h & 1) + NOps<T>::neg_if(v, h & 2);
+    return NOps<T>::add_signed(sgn(h, 0), u, sgn(h, 1), v);
 }
 template<class T> OSLMI_DEV T grad4(int hash, const T& x, const T& y, const T& z, const T& w)
 {
@@ -271,7 +289,8 @@ template<class T> OSLMI_DEV T grad4(int hash, const T& x, const T& y, const T& z
     T u   = NOps<T>::sel(h < 24, x, y);
     T v   = NOps<T>::sel(h < 16, y, z);
     T s   = NOps<T>::sel(h < 8, z, w);
-    return NOps<T>::neg_if(u, h & 1) + NOps<T>::neg_if(v, h & 2) + NOps<T>::neg_if(s, h & 4);
+    const T uv = NOps<T>::add_signed(sgn(h, 0), u, sgn(h, 1), v);
+    return NOps<T>::add_signed(sgn(h, 2), s, 1.0f, uv);
 }
 
 // Component selector of the lattice hash: shift 0 is HashScalar, 8 and 16
@@ -395,20 +414,37 @@ OSLMI_DEV uint32_t scramble(uint32_t v0, uint32_t v1, uint32_t v2)
 {
     return bjfinal(v0, v1, v2 ^ 0xdeadbeefu);
 }
-// 3D gradient table (12 cube edges + 4 repeats, sfm_simplex.h:129-183) as
-// per-component bit masks: bit i set in P/N means component = +1/-1.
+// Gradient components -1, 0 or 1 as 2-bit signed fields of a constant, so
+// a lookup is one bit-field extract and one conversion.
+// component from its masks: bit h of p / n set: +1 / -1
+constexpr uint64_t grad_fields(uint32_t p, uint32_t n, int count)
+{
+    uint64_t f = 0;
+    for (int h = 0; h < count; ++h)
+        f |= (uint64_t)(((n >> h) & 1u) ? 3u : ((p >> h) & 1u)) << (2 * h);
+    return f;
+}
+OSLMI_DEV float grad_field(uint32_t fields, uint32_t offset)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (float)(int)__builtin_amdgcn_sbfe((int)fields, offset, 2u);
+#else
+    return (float)((int32_t)(fields << (30u - offset)) >> 30);
+#endif
+}
+// 3D gradient table (12 cube edges + 4 repeats, sfm_simplex.h:129-183)
 OSLMI_DEV void simplex_grad3(uint32_t h, float g[3])
 {
-    uint32_t bit = 1u << (h & 15u);
-    g[0] = (bit & 0x1311u) ? 1.0f : ((bit & 0x2C44u) ? -1.0f : 0.0f);
-    g[1] = (bit & 0x4622u) ? 1.0f : ((bit & 0x8988u) ? -1.0f : 0.0f);
-    g[2] = (bit & 0x300Fu) ? 1.0f : ((bit & 0xC0F0u) ? -1.0f : 0.0f);
+    const uint32_t o = (h << 1) & 30u;
+    g[0] = grad_field((uint32_t)grad_fields(0x1311u, 0x2C44u, 16), o);
+    g[1] = grad_field((uint32_t)grad_fields(0x4622u, 0x8988u, 16), o);
+    g[2] = grad_field((uint32_t)grad_fields(0x300Fu, 0xC0F0u, 16), o);
 }
 OSLMI_DEV void simplex_grad2(uint32_t h, float g[2])
 {
-    uint32_t bit = 1u << (h & 7u);
-    g[0] = (bit & 0x8Au) ? 1.0f : ((bit & 0x15u) ? -1.0f : 0.0f);
-    g[1] = (bit & 0x58u) ? 1.0f : ((bit & 0xA1u) ? -1.0f : 0.0f);
+    const uint32_t o = (h << 1) & 14u;
+    g[0] = grad_field((uint32_t)grad_fields(0x8Au, 0x15u, 8), o);
+    g[1] = grad_field((uint32_t)grad_fields(0x58u, 0xA1u, 8), o);
 }
 
 OSLMI_DEV float simplex1(float x, uint32_t seed, float* dnoise)
@@ -603,11 +639,15 @@ OSLMI_DEV float simplex3(float x, float y, float z, uint32_t seed, float* dnoise
 // per-component masks over h & 31 (bit set in P / N: component +1 / -1).
 OSLMI_DEV void simplex_grad4(uint32_t h, float g[4])
 {
-    uint32_t bit = 1u << (h & 31u);
-    g[0] = (bit & 0x0F0F0F00u) ? 1.0f : ((bit & 0xF0F0F000u) ? -1.0f : 0.0f);
-    g[1] = (bit & 0x3333000Fu) ? 1.0f : ((bit & 0xCCCC00F0u) ? -1.0f : 0.0f);
-    g[2] = (bit & 0x55003333u) ? 1.0f : ((bit & 0xAA00CCCCu) ? -1.0f : 0.0f);
-    g[3] = (bit & 0x00555555u) ? 1.0f : ((bit & 0x00AAAAAAu) ? -1.0f : 0.0f);
+    const uint32_t o = (h << 1) & 30u;
+    const bool hi    = (h & 16u) != 0;
+    constexpr uint64_t f[4] = { grad_fields(0x0F0F0F00u, 0xF0F0F000u, 32),
+                                grad_fields(0x3333000Fu, 0xCCCC00F0u, 32),
+                                grad_fields(0x55003333u, 0xAA00CCCCu, 32),
+                                grad_fields(0x00555555u, 0x00AAAAAAu, 32) };
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+        g[a] = grad_field(hi ? (uint32_t)(f[a] >> 32) : (uint32_t)f[a], o);
 }
 
 // 4D simplex noise (simplexnoise4, sfm_simplex.h:970-1230). The simplex's
