@@ -58,11 +58,13 @@ std::string flit(float f)
 // six / four / three / two waves): sampled 83.8 / 66.6 / 48.6 / 59.3,
 // evaluated 42.0 / 33.6 / 22.6 / 27.5, exported (21 parameters a lobe more)
 // 80.5 / 67.3 / 43.8 / 31.2. Kernels without them run best at six (layered3,
-// 1M points: 266 us; 278, 306, 301 at five, four, three).
-std::string kernel_attributes(const ShadingSys& ss, bool mx, bool exported)
+// 1M points: 266 us; 278, 306, 301 at five, four, three). The second kernel
+// of a group with Gabor noise, launched over few points, has four: no spills,
+// and its LDS admits three.
+std::string kernel_attributes(const ShadingSys& ss, bool mx, bool exported, bool split = false)
 {
     std::string a = "__launch_bounds__(256)";
-    const int w   = ss.waves_per_eu >= 0 ? ss.waves_per_eu : !mx ? 6 : exported ? 2 : 3;
+    const int w   = ss.waves_per_eu >= 0 ? ss.waves_per_eu : !mx ? (split ? 4 : 6) : exported ? 2 : 3;
     if (w > 0)
         a += " __attribute__((amdgpu_waves_per_eu(" + std::to_string(w) + ")))";
     return a;
@@ -82,6 +84,7 @@ struct Emitter {
     int cur_layer     = 0;
     std::set<int> globals;
     bool uses_cs = false, uses_bb = false;
+    bool uses_gabor = false;
     bool uses_mx = false;  // MaterialX closures (libbsdl lobes, energy tables)
     bool uses_aniso = false;  // microfacet lobes with a tangent, two roughnesses or refraction
 
@@ -891,7 +894,8 @@ struct Emitter {
                     pp.push_back("0.0f");
                 pv = "V3(" + pp[0] + ", " + pp[1] + ", " + pp[2] + ")";
             }
-            const std::string pargs = std::string(periodic ? "true" : "false") + ", " + pv;
+            const std::string pargs = std::string(periodic ? "true" : "false") + ", " + pv + ", split_";
+            uses_gabor = true;
             line("{ const GaborUniform gu_ = " + gus + ";");
             line("  Df gx_ = " + dc[0] + ", gy_ = " + dc[1] + ", gz_ = " + dc[2] + ";");
             const std::string P = "Dv(V3(gx_.v, gy_.v, gz_.v), V3(gx_.dx, gy_.dx, gz_.dx), V3(gx_.dy, gy_.dy, gz_.dy))";
@@ -1644,6 +1648,7 @@ struct Emitter {
         code            = k.str();
         g.uses_colorsys = uses_cs;
         g.uses_mx       = uses_mx;
+        g.uses_gabor    = uses_gabor;
         g.globals_used.assign(globals.begin(), globals.end());
         return true;
     }
@@ -1657,7 +1662,19 @@ struct Emitter {
         std::ostringstream k;
         k << "// Emitted by the oslmi group emitter for group '" << g.name << "'.\n";
         k << prelude(uses_mx, g.can_export, uses_aniso);
-        k << "extern \"C\" __global__ " << kernel_attributes(ss, uses_mx, g.can_export) << " void oslmi_group_main(GroupArgs A)\n{\n";
+        kernel(k, code, false);
+        if (uses_gabor)
+            kernel(k, code, true);
+        src = k.str();
+        return true;
+    }
+
+    // One kernel over the group's points: a work-item each or, split, 64 of
+    // a workgroup's 256 (the other waves share their Gabor cells).
+    void kernel(std::ostringstream& k, const std::string& code, bool split)
+    {
+        k << "extern \"C\" __global__ " << kernel_attributes(ss, uses_mx, g.can_export, split)
+          << " void " << (split ? "oslmi_group_split" : "oslmi_group_main") << "(GroupArgs A)\n{\n";
         k << "    using Closure = LobeList<" << closure_capacity() << ">;\n";
         if (uses_cs)
             k << "    const ColorSysDev* CS = (const ColorSysDev*)A.colorsys;\n";
@@ -1666,12 +1683,16 @@ struct Emitter {
                  "    for (int j = threadIdx.x; j < OSLMI_BB_TABLE * 3; j += blockDim.x) s_bb[j] = CS->bb[j];\n"
                  "    __syncthreads();\n";
         }
-        k << "    int64_t stride = (int64_t)gridDim.x * blockDim.x;\n";
-        k << "    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < A.n; i += stride) {\n";
+        if (uses_gabor)
+            k << "    constexpr bool split_ = " << (split ? "true" : "false") << ";\n";
+        if (split)
+            k << "    int64_t stride = (int64_t)gridDim.x * 64;\n"
+                 "    for (int64_t i = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63); i < A.n; i += stride) {\n";
+        else
+            k << "    int64_t stride = (int64_t)gridDim.x * blockDim.x;\n"
+                 "    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < A.n; i += stride) {\n";
         k << code;
         k << "    }\n}\n";
-        src = k.str();
-        return true;
     }
 
     static std::string prelude(bool mx, bool xp = false, bool aniso = false)
@@ -1741,9 +1762,12 @@ bool emit_batch(const ShadingSys& ss, const std::vector<Group*>& groups,
         if (e.uses_cs)
             c << "        const ColorSysDev* CS = (const ColorSysDev*)A.colorsys;\n";
         c << "        for (;;) {\n";
+        if (e.uses_gabor)
+            c << "        constexpr bool split_ = false;\n";
         c << "#pragma unroll 1\n";
         c << "        for (int q_ = 0; q_ < B.ppt; ++q_) {\n";
-        c << "        int64_t i = T.begin + (int64_t)q_ * blockDim.x + threadIdx.x;\n";
+        c << "        int64_t i = T.begin + (int64_t)q_ * blockDim.x + "
+          << "threadIdx.x;\n";
         c << "        if (i < T.end) {\n";
         c << code;
         c << "        }\n        }\n";

@@ -267,6 +267,16 @@ struct GaborQueued {
     uint32_t state, code;  // generator state before the impulse, its cell
 };
 
+// Small launches leave most of the chip idle while each wave works through
+// its cells alone, so there a workgroup shades 64 points instead of 256: its
+// four waves run the same points side by side (`split`), each evaluates a
+// quarter of the cells, in their order, and all four add up the cells' sums,
+// in their order, from LDS. Every wave holds the same values throughout, so
+// all of them meet at the barriers. `split` is a constant of the kernel: as
+// a value it cost the other launches 12% (registers spilled in the drain).
+// Over 16,411 points (layered3, one wave per SIMD) the evaluation falls from
+// 105,000 cycles a wave to a third, the launch from 89.6 to 41.0 us.
+
 // 3039177861^k modulo 2^32: k draws of the generator at once
 constexpr uint32_t gabor_rng_pow(int k)
 {
@@ -426,7 +436,7 @@ OSLMI_DEV bool gabor_wave_box(const GaborUniform& U, V3 fl, V3 xc, GaborBox& b)
 // generator stream (0 for the scalar noise, 0/1/2 for the components of the
 // vector noise).
 OSLMI_DEV Df gabor_grid(const GaborUniform& U, const GaborPoint& gp, const Dv& P, uint32_t seed,
-                        bool periodic, V3 period)
+                        bool periodic, V3 period, bool split)
 {
     const float two_pi = 6.28318548202514648438f;
     const float two32  = 4294967296.0f;
@@ -435,7 +445,20 @@ OSLMI_DEV Df gabor_grid(const GaborUniform& U, const GaborPoint& gp, const Dv& P
     // rounding errors are below 2^-18)
     const float near2 = 1.0009765625f * two32 * two32;
     __shared__ GaborQueued queue[kGaborQueue][256];
+    extern __shared__ float split_sums[];  // [3][27][64], split launches only
     const int tid = (int)threadIdx.x;
+    // the wave's quarter of the cells
+    int wave = 0;
+    if (split) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+#endif
+        __syncthreads();  // the last evaluation's sums have been read
+        for (int k = 7 * wave; k < (wave < 3 ? 7 * wave + 7 : 27); ++k)
+            for (int c = 0; c < 3; ++c)
+                split_sums[(27 * c + k) * 64 + (tid & 63)] = 0.0f;
+        __syncthreads();
+    }
     // draws per impulse: position, direction (isotropic 2, hybrid 1), phase
     const uint32_t step = U.anisotropic == 1   ? gabor_rng_pow(4)
                           : U.anisotropic == 0 ? gabor_rng_pow(6)
@@ -453,6 +476,8 @@ OSLMI_DEV Df gabor_grid(const GaborUniform& U, const GaborPoint& gp, const Dv& P
         org = V3((float)box.ox, (float)box.oy, (float)box.oz) - fl;
     } else {
         cells = gabor_cell_mask(U, xc.v);
+        if (split)
+            cells &= 0x7fu << (7 * wave);
     }
     const V3 at = two32 * (xc.v - org) - V3(0.5f * two32);
     // the same from the centre of the cell being scanned
@@ -463,19 +488,41 @@ OSLMI_DEV Df gabor_grid(const GaborUniform& U, const GaborPoint& gp, const Dv& P
 #if defined(__HIP_DEVICE_COMPILE__)
     // per wave: the same of the wave's cell (wi, wj, wk), the cell-th of
     // ncells; and the cells cell / 64 * 64 + lane, one per lane
-    const int ncells = box.dx * box.dy * box.dz;
-    int cell = 0, wi = 0, wj = 0, wk = 0, wleft = 0, lane_count = 0;
+    int ncells = box.dx * box.dy * box.dz;
+    int cell = 0, cell0 = 0, wi = 0, wj = 0, wk = 0, wleft = 0, lane_count = 0;
     uint32_t wcode = 0, wstate = 0, lane_state = 0;
     V3 wpos = at;
+    if (split && by_wave) {
+        cell0       = cell = (wave * ncells) >> 2;
+        ncells      = ((wave + 1) * ncells) >> 2;
+        const int q = cell / box.dx;
+        wi          = cell - q * box.dx;
+        wk          = q / box.dy;
+        wj          = q - wk * box.dy;
+        wpos        = at - two32 * V3((float)wi, (float)wj, (float)wk);
+    }
 #endif
     int queued = 0, sum_code = -1;
     Df sum = Df(0.0f), cell_sum = Df(0.0f);
+    // A cell's sum is complete. An impulse in the radius lies at most one
+    // cell away from the lane's own, so the split's slot is one of 27.
+    auto close_cell = [&]() {
+        if (!split) {
+            sum = sum + cell_sum;
+        } else if (sum_code >= 0) {
+            const V3 c  = org + gabor_cell_of((uint32_t)sum_code);
+            float* slot = split_sums + (13 + (int)c.x + 3 * (int)c.y + 9 * (int)c.z) * 64 + (tid & 63);
+            slot[0]           = cell_sum.v;
+            slot[27 * 64]     = cell_sum.dx;
+            slot[2 * 27 * 64] = cell_sum.dy;
+        }
+    };
     for (;;) {
         bool last;
 #if defined(__HIP_DEVICE_COMPILE__)
         if (by_wave) {
             if (wleft <= 0 && cell < ncells) {
-                if ((cell & 63) == 0) {
+                if (((cell - cell0) & 63) == 0) {
                     const int mine = cell + (int)__lane_id();
                     const int q = mine / box.dx, k = q / box.dy;
                     GaborRng rng = gabor_cell_rng(
@@ -488,8 +535,9 @@ OSLMI_DEV Df gabor_grid(const GaborUniform& U, const GaborPoint& gp, const Dv& P
                 // left out when no lane is within a cell's width of the cell
                 if (wave_any(fmaxf(fmaxf(fabsf(wpos.x), fabsf(wpos.y)), fabsf(wpos.z))
                              < 1.50001f * two32)) {
-                    wleft   = __builtin_amdgcn_readlane(lane_count, cell & 63);
-                    wstate  = (uint32_t)__builtin_amdgcn_readlane((int)lane_state, cell & 63);
+                    const int from = (cell - cell0) & 63;
+                    wleft   = __builtin_amdgcn_readlane(lane_count, from);
+                    wstate  = (uint32_t)__builtin_amdgcn_readlane((int)lane_state, from);
                     in_cell = wpos;
                     wcode   = gabor_cell_code(wi, wj, wk);
                 }
@@ -564,7 +612,7 @@ OSLMI_DEV Df gabor_grid(const GaborUniform& U, const GaborPoint& gp, const Dv& P
                 const Dv xk = U.radius * Dv((xc.v - c) - V3(x_rng, y_rng, z_rng), xc.dx, xc.dy);
                 if (dot(xk.v, xk.v) < U.radius2) {
                     if ((int)qc != sum_code) {
-                        sum      = sum + cell_sum;
+                        close_cell();
                         cell_sum = Df(0.0f);
                         sum_code = (int)qc;
                     }
@@ -596,32 +644,40 @@ OSLMI_DEV Df gabor_grid(const GaborUniform& U, const GaborPoint& gp, const Dv& P
         if (last)
             break;
     }
-    sum = sum + cell_sum;
+    close_cell();
+    if (split) {
+        // a cell without impulses adds an exact zero
+        __syncthreads();
+        for (int k = 0; k < 27; ++k) {
+            const float* slot = split_sums + k * 64 + (tid & 63);
+            sum = sum + Df(slot[0], slot[27 * 64], slot[2 * 27 * 64]);
+        }
+    }
     return (sum * U.sqrt_lambda_inv) * U.scale;
 }
 
 // scalar_gabor / scalar_pgabor for a Dual2 point P (dim 1..3 input already
 // packed in P; pgabor pads the periods of 1 and 2 dimensions with zeros).
 OSLMI_DEV Df gabor(const GaborUniform& U, const Dv& P, bool periodic = false,
-                   V3 period = V3(0.0f))
+                   V3 period = V3(0.0f), bool split = false)
 {
     GaborPoint gp;
     gabor_setup(U, P, gp);
-    return gabor_grid(U, gp, P, 0u, periodic, period);
+    return gabor_grid(U, gp, P, 0u, periodic, period, split);
 }
 
 // scalar_gabor3 / scalar_pgabor3 (sfm_gabornoise.h:517-640): one filter
 // set-up, the three components from generator seeds 0, 1 and 2. The seed
 // loop is kept rolled: the cell walk is large and runs once per component.
 OSLMI_DEV Dv gabor3(const GaborUniform& U, const Dv& P, bool periodic = false,
-                    V3 period = V3(0.0f))
+                    V3 period = V3(0.0f), bool split = false)
 {
     GaborPoint gp;
     gabor_setup(U, P, gp);
     Df r0, r1, r2;
 #pragma clang loop unroll(disable)
     for (uint32_t seed = 0; seed < 3; ++seed) {
-        const Df r = gabor_grid(U, gp, P, seed, periodic, period);
+        const Df r = gabor_grid(U, gp, P, seed, periodic, period, split);
         if (seed == 0)
             r0 = r;
         else if (seed == 1)

@@ -69,6 +69,7 @@ struct Group {
     int output_planes        = 0;
     bool surface_closure     = false;  // some layer has the Ci global (shared by all layers)
     bool uses_colorsys       = false;
+    bool uses_gabor          = false;  // can be launched split (a workgroup shades 64 points)
     bool uses_mx             = false;  // MaterialX closures: reads the libbsdl energy tables
     bool uses_xforms         = false;  // reads the transform / attribute table
     bool can_sample          = false;  // kernel samples Ci when A.samp is set
@@ -76,6 +77,7 @@ struct Group {
     std::vector<unsigned> globals_used;  // GlobalIndex values read
     hipModule_t module       = nullptr;
     hipFunction_t kernel     = nullptr;
+    hipFunction_t split      = nullptr;  // uses_gabor: the kernel of split launches
     double jit_seconds       = 0.0;
     // oslmi_execute_wide16: symbol locations and the device workspace of
     // gathered globals and output planes (grown on demand)
@@ -175,6 +177,25 @@ int device_colorsys(const ColorSysDev** out, bool allocate = true);
 namespace mtx {
 int device_tables(const float** out, bool allocate = true);
 }
+
+// planes of each shader global
+inline constexpr int kGlobalComps[kG_COUNT] = { 3, 3, 3, 3, 3, 3, 1, 1, 1, 1, 1, 1, 1, 3, 3, 3 };
+
+// Split launches (four waves of a workgroup share 64 points' Gabor cells)
+// serve groups with Gabor noise whose outputs do not overlap their inputs.
+bool split_allowed(const Group& g, const GroupArgs& A);
+// The most points of a split launch: three workgroups of 64 points on each of
+// 256 CUs, as many as are resident at once (45 KB of LDS each). Below, one
+// wave's latency bounds the launch and the three others have idle SIMDs to
+// run on; above, the point's other work, done four times, costs more than
+// the shared scan saves. layered3 with derivatives and closure eval, us, a
+// wave's points on their own / split: 63 points 57.7 / 35.1, 4096 101.6 /
+// 46.9, 16,411 89.6 / 41.0, 32,768 81.2 / 46.1, 65,536 90.7 / 83.9, 131,072
+// 95.6 / 125.5. Of 51 generated groups with Gabor noise over 2048 unrelated
+// points 48 are faster split (216 / 137 the slowest), three alike.
+constexpr int64_t kSplitMaxPoints = 3 * 64 * 256;
+// Launches the group's own kernel over A.n > 0 points.
+int launch_group(const Group& g, GroupArgs& A, hipStream_t stream);
 
 // Kernel argument block of one execution of group g (validates the
 // arguments like BatchedExecutor::execute; `who` prefixes error messages).

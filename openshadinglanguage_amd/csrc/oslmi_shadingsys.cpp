@@ -196,6 +196,55 @@ int make_group_args(const ShadingSys& ss, const Group& g, const oslmi_batched_gl
     return OSLMI_OK;
 }
 
+bool split_allowed(const Group& g, const GroupArgs& A)
+{
+    if (!g.uses_gabor)
+        return false;
+    // The waves that shade the same points store the same values, but at
+    // different times: a buffer that is read and written at once (which one
+    // wave per point may do) is not shaded split.
+    struct Range {
+        const float* p;
+        int64_t floats;
+    };
+    Range in[kG_COUNT + 3], out[4];
+    int ni = 0, no = 0;
+    for (int k = 0; k < kG_COUNT; ++k)
+        if (A.g[k])
+            in[ni++] = { A.g[k], kGlobalComps[k] * A.n };
+    if (A.wo)
+        in[ni++] = { A.wo, 3 * A.n };
+    if (A.wi)
+        in[ni++] = { A.wi, 3 * A.n };
+    if (A.rnd)
+        in[ni++] = { A.rnd, 3 * A.n };
+    if (g.output_planes > 0)
+        out[no++] = { A.out[0], g.output_planes * A.n };
+    if (A.eval)
+        out[no++] = { A.eval, 4 * A.n };
+    if (A.samp)
+        out[no++] = { A.samp, 7 * A.n };
+    if (A.clo)
+        out[no++] = { A.clo, (1 + (int64_t)A.clo_max * OSLMI_CLOSURE_RECORD) * A.n };
+    for (int i = 0; i < ni; ++i)
+        for (int o = 0; o < no; ++o)
+            if (in[i].p < out[o].p + out[o].floats && out[o].p < in[i].p + in[i].floats)
+                return false;
+    return true;
+}
+
+int launch_group(const Group& g, GroupArgs& A, hipStream_t stream)
+{
+    void* args[] = { &A };
+    if (g.split && A.n <= kSplitMaxPoints && split_allowed(g, A))
+        return check_hip(hipModuleLaunchKernel(g.split, (unsigned)((A.n + 63) / 64), 1, 1, 256, 1, 1,
+                                               kGaborSplitLds, stream, args, nullptr),
+                         "hipModuleLaunchKernel(split)");
+    return check_hip(hipModuleLaunchKernel(g.kernel, grid_for(A.n), 1, 1, 256, 1, 1, 0, stream, args,
+                                           nullptr),
+                     "hipModuleLaunchKernel");
+}
+
 // ---- renderer services: named coordinate systems ---------------------------
 namespace {
 
@@ -354,6 +403,11 @@ int compile_group(ShadingSys& ss, Group& g, bool load = true)
     if (int rc = check_hip(hipModuleGetFunction(&g.kernel, g.module, "oslmi_group_main"),
                            "hipModuleGetFunction"))
         return rc;
+    g.split = nullptr;
+    if (g.uses_gabor)
+        if (int rc = check_hip(hipModuleGetFunction(&g.split, g.module, "oslmi_group_split"),
+                               "hipModuleGetFunction(split)"))
+            return rc;
     g.jitted = true;
     return OSLMI_OK;
 }
@@ -669,12 +723,7 @@ int oslmi_execute_batch(oslmi_shadingsys* s, oslmi_group* gh, const oslmi_batche
         return rc;
     if (bg->n == 0)
         return OSLMI_OK;
-    void* args[] = { &A };
-    if (int rc = check_hip(hipModuleLaunchKernel(g.kernel, grid_for(bg->n), 1, 1, 256, 1, 1, 0,
-                                                 (hipStream_t)stream, args, nullptr),
-                           "hipModuleLaunchKernel"))
-        return rc;
-    return OSLMI_OK;
+    return launch_group(g, A, (hipStream_t)stream);
 }
 
 int oslmi_execute_batch_sample(oslmi_shadingsys* s, oslmi_group* gh,
@@ -703,10 +752,7 @@ int oslmi_execute_batch_sample(oslmi_shadingsys* s, oslmi_group* gh,
     A.samp = d_samples;
     if (bg->n == 0)
         return OSLMI_OK;
-    void* args[] = { &A };
-    return check_hip(hipModuleLaunchKernel(g.kernel, grid_for(bg->n), 1, 1, 256, 1, 1, 0,
-                                           (hipStream_t)stream, args, nullptr),
-                     "hipModuleLaunchKernel");
+    return launch_group(g, A, (hipStream_t)stream);
 }
 
 int oslmi_execute_batch_closures(oslmi_shadingsys* s, oslmi_group* gh,
@@ -737,10 +783,7 @@ int oslmi_execute_batch_closures(oslmi_shadingsys* s, oslmi_group* gh,
     A.clo_max = max_lobes;
     if (bg->n == 0)
         return OSLMI_OK;
-    void* args[] = { &A };
-    return check_hip(hipModuleLaunchKernel(g.kernel, grid_for(bg->n), 1, 1, 256, 1, 1, 0,
-                                           (hipStream_t)stream, args, nullptr),
-                     "hipModuleLaunchKernel");
+    return launch_group(g, A, (hipStream_t)stream);
 }
 
 }  // extern "C"

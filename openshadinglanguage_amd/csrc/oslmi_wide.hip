@@ -37,7 +37,6 @@ const size_t kBsgOffset[kG_COUNT] = {
     offsetof(oslmi_bsg16, time), offsetof(oslmi_bsg16, dPdu), offsetof(oslmi_bsg16, dPdv),
     offsetof(oslmi_bsg16, Ps)
 };
-const int kGlobalComps[kG_COUNT] = { 3, 3, 3, 3, 3, 3, 1, 1, 1, 1, 1, 1, 1, 3, 3, 3 };
 
 static_assert(sizeof(oslmi_bsg16) == 4032, "BatchedShaderGlobals<16> is 4032 bytes");
 static_assert(offsetof(oslmi_bsg16, P) == 64, "VaryingShaderGlobals<16> follows a 64-byte block");
@@ -257,10 +256,7 @@ int oslmi_execute_wide16(oslmi_shadingsys* s, oslmi_group* gh, int64_t nbatch, i
     if (int rc = make_group_args(s->ss, g, &bg, outputs, nullptr, nullptr, nullptr,
                                  "oslmi_execute_wide16", A))
         return rc;
-    void* args[] = { &A };
-    if (int rc = check_hip(hipModuleLaunchKernel(g.kernel, grid_for(n), 1, 1, 256, 1, 1, 0, st, args,
-                                                 nullptr),
-                           "hipModuleLaunchKernel"))
+    if (int rc = launch_group(g, A, st))
         return rc;
     if (sp.nlocs > 0) {
         hipLaunchKernelGGL(k_symloc_scatter, dim3(grid), dim3(256), 0, st, outputs, d_shadeindex,
