@@ -311,7 +311,7 @@ typedef struct oslmi_batch_config {
 } oslmi_batch_config;
 /* Emits and compiles (hiprtc, code-object cache) the batch's persistent
  * kernels over ngroups ended groups: groups_per_kernel groups per kernel
- * (0: 8), the kernels launched one after another. load = 0 only fills the
+ * (0: the library's choice, 32), the kernels launched one after another. load = 0 only fills the
  * code-object cache (no device needed). */
 oslmi_batch* oslmi_batch_create(oslmi_shadingsys* ss, int ngroups, oslmi_group* const* groups,
                                 int groups_per_kernel, int load);

@@ -7,9 +7,8 @@
 // whenever a group has fewer points than it takes to fill it, and pays one
 // kernel's ramp-up and drain per group. A batch instead compiles the
 // groups' per-point code into a few persistent kernels ("parts", up to
-// groups_per_kernel groups each: one kernel over all groups would cost
-// minutes of compile time, and its register budget is the maximum over
-// every group, so small parts keep occupancy close to the groups' own).
+// groups_per_kernel groups each; a part's register budget is the maximum
+// over its groups, which are sorted by their need).
 // Each group's points are cut into tiles of block * ppt points; a part's
 // tile list keeps each group's tiles together (group-sorted, so
 // neighbouring workgroups run the same code) and is ordered either as given
@@ -466,7 +465,14 @@ oslmi_batch* oslmi_batch_create(oslmi_shadingsys* s, int ngroups, oslmi_group* c
         set_error(OSLMI_ERR_INVALID, "oslmi_batch_create: groups_per_kernel < 0");
         return nullptr;
     }
-    const int per = groups_per_kernel ? groups_per_kernel : 8;
+    // Few large kernels: a batch ends when its slowest tiles do, so kernels
+    // that wait for each other add up their slowest tiles, and side streams
+    // beyond the process's few hardware queues do wait. 64 generated groups,
+    // us eager (autotuned) at 8 / 16 / 32 groups per kernel: 32..2048 points
+    // each 690 / 271 / 248, 32..262,144 points 1138 / 1107 / 1069; replayed
+    // from a graph, 1155 / 736 / 408 and 1859 / 1500 / 1121. They compile in
+    // 129, 132 and 186 s; one kernel of all 64 takes 336 s, hence the limit.
+    const int per = groups_per_kernel ? groups_per_kernel : 32;
     oslmi_batch* h = new oslmi_batch;
     Batch& b       = h->b;
     b.ss           = &s->ss;
