@@ -153,11 +153,14 @@ __device__ __forceinline__ float row_sum(float v)
 // contract over samples, need them across lanes: A^T and dZ^T of one layer
 // go through LDS ([feature][sample], double buffered, one barrier a layer),
 // and each wave accumulates half of 16 gradient rows.
-// The pass of one workgroup is a chain of latencies, not of bytes or flops.
-// Measured at a batch of 16384: 21.8 us here plus 4.5 us for k_reduce_adam,
+// The pass of one workgroup is a chain of latencies, not of bytes or flops,
+// so every load is issued at the start: the weights (58 KB, written by the
+// step before) and biases come into LDS while the samples are gathered.
+// Measured at a batch of 16384: 19.4 us here plus 4.2 us for k_reduce_adam,
 // against 240 us of the former form (22 launches of one-wave GEMM tiles and
-// elementwise kernels, every activation through memory four times); four
-// waves of 32 samples instead of eight of 16 took 28.4 us.
+// elementwise kernels, every activation through memory four times); with
+// each layer's weights loaded where they are used 21.8 us, four waves of 32
+// samples instead of eight of 16 28.4 us.
 // idx (optional): sample k of the batch is column idx[k] of the planes (one
 // outside them counts as no sample). part: [workgroup][NPARAM] partial
 // gradients; lpart: [workgroup] sums of squared errors.
@@ -170,6 +173,8 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_fwd_bwd(
 {
     __shared__ __align__(16) bf16 s_z[2][H][LDT], s_a[2][H][LDT];
     __shared__ float s_b[TRAIN_WAVES][4 * H + 16], s_l[TRAIN_WAVES];
+    __shared__ bf16x8 s_w[(NFWD + NBWD) * 64];
+    __shared__ __align__(16) float s_bias[4 * H + 16];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int g = lane >> 4, r = lane & 15;
     const int col = wv * 16 + r;  // this lane's column of the workgroup's 128
@@ -177,22 +182,53 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_fwd_bwd(
     const int smp = blockIdx.x * TRAIN_ROWS + col;
     bool live     = smp < B;
     int64_t src   = live ? (idx ? idx[smp] : smp) : 0;
+    // all weights, on their way while the samples are gathered
+    constexpr int kFrags = ((NFWD + NBWD) * 64 + 64 * TRAIN_WAVES - 1) / (64 * TRAIN_WAVES);
+    bf16x8 frag[kFrags];
+#pragma unroll
+    for (int k = 0; k < kFrags; k++) {
+        const int e = 64 * TRAIN_WAVES * k + (int)threadIdx.x;
+        if (e < (NFWD + NBWD) * 64)
+            frag[k] = e < NFWD * 64 ? fwd[e] : bwd[e - NFWD * 64];
+    }
+    float bias = 0.0f;
+    if (threadIdx.x < 4 * H + 16) {
+        const int l = threadIdx.x / H;
+        bias        = P[(l < 4 ? OFF_B[1] + l * (OFF_B[2] - OFF_B[1]) : OFF_B[5]) + threadIdx.x % H];
+    }
+    float off[8], scl[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const int k = 8 * g + j < NIN ? 8 * g + j : 0;
+        off[j]      = nm.in_off[k];
+        scl[j]      = nm.in_scale[k];
+    }
     if (src < 0 || src >= ldq) {
         live = false;
         src  = 0;
     }
-    bf16x8 x;
+    float xin[8], raw[NOUT];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int k   = 8 * g + j;
-        const int kc  = k < NIN ? k : 0;
-        const float v = (q[kc * ldq + src] - nm.in_off[kc]) * nm.in_scale[kc];
-        x[j]          = (bf16)(k < NIN && live ? v : 0.0f);
-    }
-    float raw[NOUT];
+    for (int j = 0; j < 8; j++)
+        xin[j] = q[(8 * g + j < NIN ? 8 * g + j : 0) * ldq + src];
 #pragma unroll
     for (int o = 0; o < NOUT; o++)
         raw[o] = t[o * ldq + src];
+#pragma unroll
+    for (int k = 0; k < kFrags; k++)
+        if (64 * TRAIN_WAVES * k + (int)threadIdx.x < (NFWD + NBWD) * 64)
+            s_w[64 * TRAIN_WAVES * k + threadIdx.x] = frag[k];
+    if (threadIdx.x < 4 * H + 16)
+        s_bias[threadIdx.x] = bias;
+    const bf16x8* lfwd = s_w + lane;
+    const bf16x8* lbwd = s_w + NFWD * 64 + lane;
+    bf16x8 x;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const float v = (xin[j] - off[j]) * scl[j];
+        x[j]          = (bf16)(8 * g + j < NIN && live ? v : 0.0f);
+    }
+    __syncthreads();
     // forward: h[l] layer l's activations (B operands), d[l] SiLU'
     bf16x8 h[5][2];
     f32x4 d[5][4];
@@ -201,15 +237,15 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_fwd_bwd(
         f32x4 acc[4];
 #pragma unroll
         for (int m = 0; m < 4; m++) {
-            const f32x4 b = *reinterpret_cast<const f32x4*>(P + OFF_B[l] + 16 * m + 4 * g);
+            const f32x4 b = *reinterpret_cast<const f32x4*>(s_bias + (l - 1) * H + 16 * m + 4 * g);
             if (l == 1) {
-                acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fwd[(FWD_OF[1] + m) * 64 + lane],
+                acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lfwd[(FWD_OF[1] + m) * 64],
                                                                  x, b, 0, 0, 0);
             } else {
                 acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    fwd[(FWD_OF[l] + 2 * m) * 64 + lane], h[l - 1][0], b, 0, 0, 0);
+                    lfwd[(FWD_OF[l] + 2 * m) * 64], h[l - 1][0], b, 0, 0, 0);
                 acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    fwd[(FWD_OF[l] + 2 * m + 1) * 64 + lane], h[l - 1][1], acc[m], 0, 0, 0);
+                    lfwd[(FWD_OF[l] + 2 * m + 1) * 64], h[l - 1][1], acc[m], 0, 0, 0);
             }
         }
 #pragma unroll
@@ -224,9 +260,9 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_fwd_bwd(
     }
     // output layer, loss, and its gradient 2 (pred - y) / (4 B): lanes of
     // group 0 hold the four outputs
-    f32x4 out = *reinterpret_cast<const f32x4*>(P + OFF_B[5] + 4 * g);
-    out = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fwd[FWD_OF[5] * 64 + lane], h[4][0], out, 0, 0, 0);
-    out = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fwd[(FWD_OF[5] + 1) * 64 + lane], h[4][1], out, 0, 0, 0);
+    f32x4 out = *reinterpret_cast<const f32x4*>(s_bias + 4 * H + 4 * g);
+    out = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lfwd[FWD_OF[5] * 64], h[4][0], out, 0, 0, 0);
+    out = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lfwd[(FWD_OF[5] + 1) * 64], h[4][1], out, 0, 0, 0);
     const float scale = 2.0f / (4.0f * (float)B);
     float lsum = 0.0f;
     bf16x8 z[2];  // dZ of the layer as B operand
@@ -275,9 +311,9 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_fwd_bwd(
             for (int m = 0; m < 4; m++) {
                 const int f = BWD_OF[l] + (l == 5 ? m : 2 * m);
                 f32x4 acc   = { 0.0f, 0.0f, 0.0f, 0.0f };
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bwd[f * 64 + lane], z[0], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lbwd[f * 64], z[0], acc, 0, 0, 0);
                 if (l < 5)
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bwd[(f + 1) * 64 + lane], z[1], acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lbwd[(f + 1) * 64], z[1], acc, 0, 0, 0);
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     const float v                  = acc[j] * d[l - 1][m][j];
