@@ -59,12 +59,12 @@ std::string flit(float f)
 // evaluated 42.0 / 33.6 / 22.6 / 27.5, exported (21 parameters a lobe more)
 // 80.5 / 67.3 / 43.8 / 31.2. Kernels without them run best at six (layered3,
 // 1M points: 266 us; 278, 306, 301 at five, four, three). The second kernel
-// of a group with Gabor noise, launched over few points, has four: no spills,
-// and its LDS admits three.
+// of a group with Gabor noise, launched over few points, has the three that
+// its LDS (45 KB) admits, and no spills.
 std::string kernel_attributes(const ShadingSys& ss, bool mx, bool exported, bool split = false)
 {
     std::string a = "__launch_bounds__(256)";
-    const int w   = ss.waves_per_eu >= 0 ? ss.waves_per_eu : !mx ? (split ? 4 : 6) : exported ? 2 : 3;
+    const int w   = ss.waves_per_eu >= 0 ? ss.waves_per_eu : !mx ? (split ? 3 : 6) : exported ? 2 : 3;
     if (w > 0)
         a += " __attribute__((amdgpu_waves_per_eu(" + std::to_string(w) + ")))";
     return a;

@@ -44,10 +44,6 @@ struct GroupArgs {
     int32_t clo_pad;
 };
 
-// Dynamic LDS of a split launch: a value and two derivatives for the 27
-// Gabor cells around each of 64 points.
-constexpr int kGaborSplitLds = 27 * 64 * 3 * 4;
-
 // planes per exported lobe: id, weight rgb, 21 parameter floats (the
 // largest set, generalized_schlick_bsdf's)
 #define OSLMI_CLOSURE_PARAMS 21

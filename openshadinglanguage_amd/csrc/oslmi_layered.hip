@@ -26,10 +26,11 @@
 
 // Workgroup sizes of the layered-closure kernels. Each workgroup stages the
 // 33 KB energy tables in LDS, so at most four workgroups fit on a CU. The
-// eval+sample kernel needs 119 registers (four waves per SIMD), which 256
-// work-items per workgroup already reach; the eval-only kernels need about
-// 84, and 512 work-items per workgroup let five or six waves per SIMD share
-// one copy of the tables (6 % faster over 8M queries than 256).
+// eval+sample kernel needs 113 registers, 128 with a base roughness of its
+// own (four waves per SIMD), which 256 work-items per workgroup already
+// reach; the eval-only kernels hold 8 KB of queued queries besides, and two
+// workgroups of 512 work-items give four waves per SIMD, three of 256 three
+// (512 measured 6 % faster over 8M queries).
 constexpr int kLayeredBlock = 256;
 constexpr int kLocalBlock   = 512;
 

@@ -3,7 +3,7 @@
 // One work-item evaluates one shading point; the batched CPU path's W=16
 // lane loop becomes the 64-wide wavefront. Perlin/cell/hash noise use no
 // tables at all (pure integer VALU work: the Jenkins hash below); simplex
-// uses a 16-entry gradient table held in registers as bit masks.
+// gradient components are two-bit fields of constants.
 //
 // Reference algorithms (file:line in the reference tree):
 //   bjmix/bjfinal               src/include/OSL/oslnoise.h:154-180

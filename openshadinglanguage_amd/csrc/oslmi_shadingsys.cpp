@@ -237,8 +237,8 @@ int launch_group(const Group& g, GroupArgs& A, hipStream_t stream)
 {
     void* args[] = { &A };
     if (g.split && A.n <= kSplitMaxPoints && split_allowed(g, A))
-        return check_hip(hipModuleLaunchKernel(g.split, (unsigned)((A.n + 63) / 64), 1, 1, 256, 1, 1,
-                                               kGaborSplitLds, stream, args, nullptr),
+        return check_hip(hipModuleLaunchKernel(g.split, (unsigned)((A.n + 63) / 64), 1, 1, 256, 1, 1, 0,
+                                               stream, args, nullptr),
                          "hipModuleLaunchKernel(split)");
     return check_hip(hipModuleLaunchKernel(g.kernel, grid_for(A.n), 1, 1, 256, 1, 1, 0, stream, args,
                                            nullptr),
