@@ -251,7 +251,8 @@ OSLMI_DEV Df gabor_impulse(const GaborUniform& U, const GaborPoint& gp, V3 omega
 //
 // What is left is the scan, which has two forms:
 //  * per wave: the 64 lanes shade neighbouring points, whose cells fill a
-//    small box (at most 8 x 8 x 4 and 128 cells, every lane active). Each
+//    small box (at most 8 x 8 x 4 and 128 cells, every lane active; the
+//    periods of a periodic noise, which wrap the cells, all alike). Each
 //    lane seeds the generator of one of the box's cells and draws its
 //    impulse count; then all lanes test every impulse of the box together.
 //    The generator runs once per wave, in the scalar unit, and nothing
@@ -408,6 +409,20 @@ template<bool MAX> OSLMI_DEV int wave_extreme(int v)
 }
 #endif
 
+// Whether every active lane of the wave holds the same vector, bit for bit.
+OSLMI_DEV bool wave_same(V3 v)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    const uint32_t x = __float_as_uint(v.x), y = __float_as_uint(v.y), z = __float_as_uint(v.z);
+    return !wave_any(x != (uint32_t)__builtin_amdgcn_readfirstlane((int)x)
+                     || y != (uint32_t)__builtin_amdgcn_readfirstlane((int)y)
+                     || z != (uint32_t)__builtin_amdgcn_readfirstlane((int)z));
+#else
+    (void)v;
+    return true;
+#endif
+}
+
 // The wave's box of cells: origin (ox, oy, oz), size (dx, dy, dz). False
 // where the per-wave scan does not apply. An axis reaches one cell beyond
 // the lanes' own cells on either side, above only where a lane needs it.
@@ -475,7 +490,9 @@ OSLMI_DEV Df gabor_grid(const GaborUniform& U, const GaborPoint& gp, const Dv& P
     V3 fl(floorf(xg.v.x), floorf(xg.v.y), floorf(xg.v.z));
     Dv xc(xg.v - fl, xg.dx, xg.dy);
     GaborBox box = { 0, 0, 0, 0, 0, 0 };
-    const bool by_wave = gabor_wave_box(U, fl, xc.v, box);
+    // a wave's cells are wrapped and seeded once, so by one period: points
+    // with periods of their own walk their own cells
+    const bool by_wave = gabor_wave_box(U, fl, xc.v, box) && (!periodic || wave_same(period));
     // the queued cells' origin relative to this lane's cell, and the lane's
     // position from that cell's centre in units of 2^-32 cells
     V3 org(-1.0f, -1.0f, -1.0f);
