@@ -448,6 +448,16 @@ struct Emitter {
         return k >= 0 && S(L, k).kind == kGlobal && S(L, k).type.base == kClosure ? k : -1;
     }
 
+    // (layer, symbol) of an output name: "layer.symbol", or a symbol of any
+    // layer. The symbol may be a structure's member, with a dot of its own.
+    static std::pair<std::string, std::string> output_parts(const std::string& on)
+    {
+        const size_t dot = on.find('.');
+        if (dot == std::string::npos)
+            return { "", on };
+        return { on.substr(0, dot), on.substr(dot + 1) };
+    }
+
     // Symbols whose value can reach a renderer output, a closure or a branch
     // (flow-insensitive: a symbol counts as read by every op that may write
     // a live one). The compiler drops dead arithmetic by itself, but not a
@@ -470,7 +480,7 @@ struct Emitter {
             for (size_t s = 0; s < m.syms.size(); ++s) {
                 bool root = m.syms[s].kind == kGlobal;
                 for (const std::string& o : g.output_names)
-                    root = root || o.substr(o.find_last_of('.') + 1) == m.syms[s].name;
+                    root = root || output_parts(o).second == m.syms[s].name;
                 if (root)
                     mark((int)L, (int)s);
             }
@@ -1489,12 +1499,7 @@ struct Emitter {
         g.outputs.clear();
         int plane = 0;
         for (const std::string& on : g.output_names) {
-            std::string ln, sn = on;
-            size_t dot = on.find('.');
-            if (dot != std::string::npos) {
-                ln = on.substr(0, dot);
-                sn = on.substr(dot + 1);
-            }
+            const auto [ln, sn] = output_parts(on);
             int L = -1, s = -1;
             for (int k = (int)g.layers.size() - 1; k >= 0 && L < 0; --k) {
                 if (!ln.empty() && g.layers[k].name != ln)

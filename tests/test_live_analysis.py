@@ -47,6 +47,18 @@ def test_unread_gabor_is_left_out():
         assert "gabor(gu_" in ss.emit(gg)
 
 
+def test_gabor_of_a_structure_member_output_is_emitted():
+    """An output may be a structure's member, whose name holds a dot."""
+    o = G.Oso("surface", "member")
+    o.sym("global", "point", "P")
+    o.sym("oparam", "float", "out.val", "0")
+    o.op("noise", "out.val", o.const("string", "gabor"), "P")
+    ss = S.ShadingSystem()
+    g = S.build_generated_group(ss, ([("member", "surface", o.text())], []), "member",
+                                outputs=["surface.out.val"])
+    assert "gabor(gu_" in ss.emit(g)
+
+
 def test_occupancy_target_by_kernel():
     """Unset, the target follows the kernel's closures; a set one holds."""
     for mode, want in ((None, 3), ("closure_sample", 3), ("closure_export", 2)):
