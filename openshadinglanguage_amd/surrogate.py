@@ -144,16 +144,19 @@ class Surrogate:
         for x in (queries, targets):
             if not x.is_cuda or x.dtype != torch.float32:
                 raise ValueError("train needs float32 CUDA tensors")
-        # the step reads whole planes of n values; other strides are copied once
-        queries, targets = queries.contiguous(), targets[:, :n].contiguous()
         gen = torch.Generator(device=queries.device)
         gen.manual_seed(seed)
-        stream = stream or torch.cuda.current_stream()
+        caller = torch.cuda.current_stream()
+        stream = stream or caller
         sp = ctypes.c_void_p(stream.cuda_stream)
         t0 = time.perf_counter()
         log = []
-        pq, pt = _p(queries), _p(targets)
+        stream.wait_stream(caller)  # what the caller has queued on the tensors
         with torch.cuda.stream(stream):
+            # the step reads whole planes of n values; other strides are
+            # copied once, on the stream that reads the copies
+            queries, targets = queries.contiguous(), targets[:, :n].contiguous()
+            pq, pt = _p(queries), _p(targets)
             for k in range(steps):
                 idx = torch.randint(0, n, (batch,), device=queries.device, generator=gen)
                 self.step += 1

@@ -81,6 +81,11 @@ def test_train_takes_strided_planes_and_refuses_others(data):
     a.train(q[:, :4096].contiguous(), t[:, :4096].contiguous(), 4, batch=256)
     b.train(q[:, :4096], t[:, :4096], 4, batch=256)  # rows 8192 apart
     assert np.array_equal(a.get_params(), b.get_params())
+    # the copies that other strides need, on a stream of the caller's; t has
+    # more columns than samples
+    c = _surrogate()
+    c.train(q[:, :4096], t, 4, batch=256, stream=torch.cuda.Stream())
+    assert np.array_equal(a.get_params(), c.get_params())
     for bad in ((q.double(), t), (q, t[:, :100]), (q[:13], t), (q.cpu(), t.cpu())):
         with pytest.raises(ValueError):
             a.train(*bad, 1, batch=256)
