@@ -134,12 +134,13 @@ class Surrogate:
 
     def train(self, queries, targets, steps, batch=16384, lr=2e-3, lr_min=1e-5, seed=0,
               log_every=0, stream=None, progress=None):
-        """Minibatch Adam over device planes queries [14, n], targets [4, n].
+        """Minibatch Adam over device planes queries [14, n], targets [4, n]
+        (planes and targets beyond these are not read).
         progress(k) (optional) is called every 2000 steps."""
         import torch
         n = queries.shape[1]
-        if (tuple(queries.shape) != (NIN, n) or targets.dim() != 2 or targets.shape[0] != NOUT
-                or targets.shape[1] < n):
+        if (queries.dim() != 2 or queries.shape[0] < NIN or targets.dim() != 2
+                or targets.shape[0] < NOUT or targets.shape[1] < n):
             raise ValueError("train needs queries [14, n] and targets [4, n]")
         for x in (queries, targets):
             if not x.is_cuda or x.dtype != torch.float32:

@@ -86,6 +86,10 @@ def test_train_takes_strided_planes_and_refuses_others(data):
     c = _surrogate()
     c.train(q[:, :4096], t, 4, batch=256, stream=torch.cuda.Stream())
     assert np.array_equal(a.get_params(), c.get_params())
+    # planes beyond the 14 and 4 are not read
+    d = _surrogate()
+    d.train(torch.cat([q, q[:2]])[:, :4096], torch.cat([t, t[:1]]), 4, batch=256)
+    assert np.array_equal(a.get_params(), d.get_params())
     for bad in ((q.double(), t), (q, t[:, :100]), (q[:13], t), (q.cpu(), t.cpu())):
         with pytest.raises(ValueError):
             a.train(*bad, 1, batch=256)
