@@ -122,12 +122,13 @@ __global__ __launch_bounds__(256) void k_pack_train(const float* __restrict__ P,
     }
 }
 
-// SiLU and its derivative from one sigmoid. exp2 and reciprocal are the
-// hardware's, about 1 ulp each; the activations are rounded to bf16 next.
+// SiLU and its derivative. expf and IEEE divisions: the derivative scales
+// the fp32 gradient, whose sums over the samples are the bias gradients.
 __device__ __forceinline__ void silu_both(float z, float* a, float* da)
 {
-    const float s = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * z));
-    *a            = z * s;
+    const float d = 1.0f + expf(-z);
+    const float s = 1.0f / d;
+    *a            = z / d;
     *da           = s * (1.0f + z * (1.0f - s));
 }
 
@@ -156,11 +157,12 @@ __device__ __forceinline__ float row_sum(float v)
 // The pass of one workgroup is a chain of latencies, not of bytes or flops,
 // so every load is issued at the start: the weights (58 KB, written by the
 // step before) and biases come into LDS while the samples are gathered.
-// Measured at a batch of 16384: 19.4 us here plus 4.2 us for k_reduce_adam,
+// Measured at a batch of 16384: 25.7 us here plus 4.6 us for k_reduce_adam,
 // against 240 us of the former form (22 launches of one-wave GEMM tiles and
-// elementwise kernels, every activation through memory four times); with
-// each layer's weights loaded where they are used 21.8 us, four waves of 32
-// samples instead of eight of 16 28.4 us.
+// elementwise kernels, every activation through memory four times). 6.3 us
+// of it are the SiLU's expf and divisions; with the hardware's exp2 and
+// reciprocal in their place 19.4 us, and 21.8 where each layer's weights were
+// loaded where they are used, 28.4 with four waves of 32 samples.
 // idx (optional): sample k of the batch is column idx[k] of the planes (one
 // outside them counts as no sample). part: [workgroup][NPARAM] partial
 // gradients; lpart: [workgroup] sums of squared errors.

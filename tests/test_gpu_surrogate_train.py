@@ -93,3 +93,34 @@ def test_train_takes_strided_planes_and_refuses_others(data):
     for bad in ((q.double(), t), (q, t[:, :100]), (q[:13], t), (q.cpu(), t.cpu())):
         with pytest.raises(ValueError):
             a.train(*bad, 1, batch=256)
+
+
+def test_activation_derivative_keeps_binary32_accuracy(data):
+    """Layer 1 with zero weights: every sample has the biases as its
+    pre-activations, and layer 2 weighs all units alike, so the units' bias
+    gradients stand in the ratio of their SiLU derivatives (to 0.5, that of a
+    unit at zero). Bound, relative: exp 1 ulp (2^-23), the sum, the quotient,
+    four operations of the derivative and two inexact adds of 64 equal terms
+    2^-24 each, the last factor for the reference unit: 12 * 2^-24. The
+    biases are ones whose product with log2(e) rounds badly: an exponential
+    of that product is off by 20 * 2^-24 there."""
+    B = 64
+    z = np.linspace(-30, -22.5, 100000).astype(np.float32)
+    prod = (z * np.float32(1.4426950408889634)).astype(np.float64)
+    z = z[np.argsort(-np.abs(prod - z.astype(np.float64) * 1.4426950408889634))[:63]]
+    z = np.concatenate([[0.0], z]).astype(np.float32)
+    p = M.unpack(S.init_params(7).astype(np.float64))
+    p["W1"][:] = 0.0
+    p["b1"][:] = z
+    p["W2"][:] = p["W2"][:, :1]
+    q = data[0][:, :B].contiguous()
+    t = torch.full((4, B), 50.0, device="cuda:0")  # errors of one sign
+    s = _surrogate()
+    s.set_params(M.pack(p).astype(np.float32))
+    print("bias gradients, batch %d" % B, flush=True)
+    g, _ = s.grads(q, t)
+    g = M.unpack(g.astype(np.float64))["b1"]
+    sg = 1 / (1 + np.exp(-z.astype(np.float64)))
+    want = sg * (1 + z.astype(np.float64) * (1 - sg))
+    assert g[0] != 0
+    assert np.abs(g / g[0] * 0.5 / want - 1).max() <= 12 * 2.0 ** -24
