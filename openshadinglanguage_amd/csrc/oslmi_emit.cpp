@@ -256,6 +256,30 @@ struct Emitter {
         ncoord = is_periodic_noise(op.name) ? n / 2 : n;
     }
 
+    // Options of a Gabor noise: the (name, value) pairs from argument `a` on
+    GaborOptions gabor_options(int L, const OOp& op, size_t a)
+    {
+        GaborOptions go;
+        for (; a + 1 < op.args.size(); a += 2) {
+            std::string key;
+            strval(L, op.args[a], key);
+            std::vector<float> v;
+            numval(L, op.args[a + 1], v);
+            if (v.empty())
+                v.push_back(0.0f);
+            if (key == "anisotropic") go.anisotropic = (int)v[0];
+            else if (key == "do_filter") go.do_filter = (int)v[0];
+            else if (key == "bandwidth") go.bandwidth = v[0];
+            else if (key == "impulses") go.impulses = v[0];
+            else if (key == "direction" && v.size() >= 3) {
+                go.direction[0] = v[0];
+                go.direction[1] = v[1];
+                go.direction[2] = v[2];
+            }
+        }
+        return go;
+    }
+
     bool differentiable(const std::string& o)
     {
         static const std::set<std::string> d = {
@@ -571,6 +595,142 @@ struct Emitter {
         }
     }
 
+    // ---- the work of a point, for the rule of split launches ----------
+    // In units of a scalar perlin or simplex noise (about 0.4 us of a wave
+    // alone on its SIMD): the impulses of the Gabor noises, those that not
+    // every point evaluates at 1/32, and everything else that is read,
+    // counted high (both sides of a branch, closures as evaluated).
+    struct Work {
+        double impulses = 0, rest = 0;
+        bool every      = true;   // every point runs the ops walked now
+        bool left       = false;  // a point may have left the code walked so far
+    };
+    static constexpr double kUnknownWork = 1e9;
+
+    // Value of a symbol that is the same in every point and never written
+    bool constant(int L, int s, double& v)
+    {
+        const OSymbol& y = S(L, s);
+        if (y.kind != kConst && y.kind != kParam)
+            return false;
+        for (const Connection& c : g.conns)
+            if (c.dst_layer == L && c.dst_sym == s)
+                return false;
+        for (const OOp& op : M(L).ops)
+            if (!op.args.empty() && op.args[0] == s)
+                return false;
+        std::vector<float> f;
+        if (!numval(L, s, f) || f.empty())
+            return false;
+        v = f[0];
+        return true;
+    }
+
+    // Rounds of for (i = a; i < b; i += c) with constants a, b, c; negative
+    // for any other loop
+    double rounds(int L, const OOp& loop, int b)
+    {
+        const std::vector<OOp>& ops = M(L).ops;
+        const int j0 = loop.jump[0], j1 = loop.jump[1], j2 = loop.jump[2], j3 = loop.jump[3];
+        if (loop.name != "for" || j1 != j0 + 1 || j3 != j2 + 1 || j0 <= b)
+            return -1;
+        const OOp &cond = ops[j0], &step = ops[j2];
+        if ((cond.name != "lt" && cond.name != "le") || cond.args.size() != 3
+            || cond.args[0] != loop.args[0] || step.name != "add" || step.args.size() != 3)
+            return -1;
+        const int i = cond.args[1];
+        double from = 0, to, by;
+        if (step.args[0] != i || step.args[1] != i || !constant(L, step.args[2], by) || by <= 0
+            || !constant(L, cond.args[2], to))
+            return -1;
+        bool set = false;
+        for (int k = b; k < j0; ++k)
+            if (ops[k].name == "assign" && ops[k].args[0] == i)
+                set = constant(L, ops[k].args[1], from);
+        for (int k = j1; k < j2; ++k)
+            if (!ops[k].args.empty() && ops[k].args[0] == i)
+                return -1;
+        return set ? std::max(0.0, std::ceil((to - from) / by) + (cond.name == "le")) : -1;
+    }
+
+    void walk_work(int L, int b, int e, double times, Work& w)
+    {
+        const std::vector<OOp>& ops = M(L).ops;
+        for (int i = b; i < e;) {
+            const OOp& op    = ops[i];
+            const bool every = w.every;
+            if (op.name == "if") {
+                w.every = false;
+                walk_work(L, i + 1, op.jump[1], times, w);
+                i = op.jump[1];
+            } else if (op.name == "for" || op.name == "while" || op.name == "dowhile") {
+                const double n = rounds(L, op, i + 1);
+                if (n < 0)
+                    w.rest += kUnknownWork;
+                walk_work(L, i + 1, op.jump[0], times, w);
+                w.every = w.every && n >= 0;
+                walk_work(L, op.jump[0], op.jump[3], n >= 0 ? times * n : times, w);
+                i = op.jump[3];
+            } else if (op.name == "functioncall") {
+                walk_work(L, i + 1, op.jump[0], times, w);
+                i = op.jump[0];
+            } else {
+                if (op.name == "break" || op.name == "continue" || op.name == "exit" || op.name == "return")
+                    w.left = true;
+                else
+                    count_op(L, op, times, w);
+                ++i;
+            }
+            w.every = every && !w.left;
+        }
+    }
+
+    void count_op(int L, const OOp& op, double times, Work& w)
+    {
+        const std::string& o = op.name;
+        if ((is_noise_op(o) || o == "closure") && !live[L][op.args[0]])
+            return;
+        if (is_noise_op(o)) {
+            std::string nm;
+            int first, nc, nnum, dim = 0;
+            noise_layout(L, op, nm, first, nc, &nnum);
+            const Kind k       = kind(L, op.args[0]);
+            const double three = k == K_V3 || k == K_DV ? 3 : 1;
+            if (nm == "gabor") {
+                w.impulses += times * three * (w.every ? 1 : 1.0 / 32)
+                              * std::min(std::max(gabor_options(L, op, first + nnum).impulses, 1.0f), 32.0f);
+                return;
+            }
+            for (int a = 0; a < nc; ++a)
+                dim += S(L, op.args[first + a]).type.base == kTriple ? 3 : 1;
+            const bool cell = nm == "cell" || nm == "cellnoise" || nm == "hash" || nm == "hashnoise";
+            w.rest += times * three * (cell ? 0.25 : 1) * (dim == 4 ? 2 : 1)
+                      * (!cell && (k == K_DF || k == K_DV) ? 2.5 : 1);
+        } else if (o == "closure") {
+            std::string cname;
+            strval(L, op.args[1], cname);
+            const double lobe = cname == "layer" ? 0 : cname.find("_bsdf") != std::string::npos ? 6
+                                : cname == "microfacet" ? (uses_aniso ? 4 : 2) : 1;
+            w.rest += times * lobe * (ss.closure_sample ? 1.5 : 1);
+        } else {
+            w.rest += times * (o == "blackbody" || o == "transformc" ? 1 : o == "useparam" ? 0 : 0.05);
+        }
+    }
+
+    // The most points of a split launch of the group
+    int64_t split_points()
+    {
+        Work w;
+        for (int L = 0; L < (int)g.layers.size(); ++L) {
+            w.every = true;
+            w.left  = false;
+            walk_work(L, M(L).main_begin, (int)M(L).ops.size(), 1, w);
+        }
+        return w.rest <= 2.5 * w.impulses ? kSplitPoints[2]
+               : w.rest <= 4 * w.impulses ? kSplitPoints[1]
+                                          : kSplitPoints[0];
+    }
+
     // ----------------------------------------------------------- codegen
     void line(const std::string& s) { os << "        " << s << "\n"; }
 
@@ -856,25 +1016,7 @@ struct Emitter {
         if (nm == "gabor" && !live[L][r])
             return;
         if (nm == "gabor") {
-            GaborOptions go;
-            for (size_t a = first + nnum; a + 1 < op.args.size(); a += 2) {
-                std::string key;
-                strval(L, op.args[a], key);
-                std::vector<float> v;
-                numval(L, op.args[a + 1], v);
-                if (v.empty())
-                    v.push_back(0.0f);
-                if (key == "anisotropic") go.anisotropic = (int)v[0];
-                else if (key == "do_filter") go.do_filter = (int)v[0];
-                else if (key == "bandwidth") go.bandwidth = v[0];
-                else if (key == "impulses") go.impulses = v[0];
-                else if (key == "direction" && v.size() >= 3) {
-                    go.direction[0] = v[0];
-                    go.direction[1] = v[1];
-                    go.direction[2] = v[2];
-                }
-            }
-            GaborUniform gu = build_gabor_uniform(go);
+            GaborUniform gu = build_gabor_uniform(gabor_options(L, op, first + nnum));
             std::string gus = "GaborUniform{" + flit(gu.a) + "," + flit(gu.lambda) + ","
                               + flit(gu.sqrt_lambda_inv) + "," + flit(gu.radius) + ","
                               + flit(gu.radius2) + "," + flit(gu.radius3) + "," + flit(gu.radius_inv)
@@ -1668,8 +1810,11 @@ struct Emitter {
         k << "// Emitted by the oslmi group emitter for group '" << g.name << "'.\n";
         k << prelude(uses_mx, g.can_export, uses_aniso);
         kernel(k, code, false);
-        if (uses_gabor)
+        if (uses_gabor) {
+            g.split_points = split_points();
+            k << "// split launches: up to " << g.split_points << " points\n";
             kernel(k, code, true);
+        }
         src = k.str();
         return true;
     }

@@ -56,6 +56,26 @@ struct SymLoc {
     int64_t offset = 0, stride = 0;
 };
 
+// The most points of a split launch, by what the group does besides its
+// Gabor noises (split_points in the emitter): workgroups of 64 points on half
+// of the 256 CUs, two on each, three on each (as many as are resident, 45 KB
+// of LDS each). Below the first, one wave's latency bounds the launch and
+// the three others have idle SIMDs; above, the point's other work, done four
+// times, takes issue slots, 1.6 times a wave's own time at two workgroups a
+// CU and 2.2 at three, and has to be small against what sharing the cells
+// saves. Measured, us, split / a work-item each, at 8192, 32,768 and 49,152
+// points; w: work besides, in scalar noises per impulse of the Gabor noises:
+//   layered3 (w 2.0)                          47 / 97, 47 / 81, 60 / 85
+//   12 vector noises, 16 impulses (w 2.4)     40 / 69, 52 / 67, 63 / 67
+//   8 vector noises, 8 impulses (w 3.3)       26 / 46, 34 / 45, 44 / 44
+//   12 vector noises, 8 impulses (w 4.9)      30 / 50, 42 / 49, 56 / 48
+//   three MaterialX lobes, 4 impulses (w 4.8) 23 / 30, 28 / 31, 37 / 30
+//   12 vector noises, 4 impulses (w 9.8)      24 / 35, 36 / 35, 48 / 34
+//   24 vector noises, 1 impulse (w 76)        36 / 38, 54 / 36, 77 / 36
+// A Gabor noise that only some points evaluate counts 1/32: it may be nearly
+// free, as may the launch around it.
+inline constexpr int64_t kSplitPoints[3] = { 64 * 128, 2 * 64 * 256, 3 * 64 * 256 };
+
 struct Group {
     std::string name;
     bool ended = false;
@@ -78,6 +98,7 @@ struct Group {
     hipModule_t module       = nullptr;
     hipFunction_t kernel     = nullptr;
     hipFunction_t split      = nullptr;  // uses_gabor: the kernel of split launches
+    int64_t split_points     = 0;        // and the most points of one
     double jit_seconds       = 0.0;
     // oslmi_execute_wide16: symbol locations and the device workspace of
     // gathered globals and output planes (grown on demand)
@@ -184,16 +205,6 @@ inline constexpr int kGlobalComps[kG_COUNT] = { 3, 3, 3, 3, 3, 3, 1, 1, 1, 1, 1,
 // Split launches (four waves of a workgroup share 64 points' Gabor cells)
 // serve groups with Gabor noise whose outputs do not overlap their inputs.
 bool split_allowed(const Group& g, const GroupArgs& A);
-// The most points of a split launch: three workgroups of 64 points on each of
-// 256 CUs, as many as are resident at once (45 KB of LDS each). Below, one
-// wave's latency bounds the launch and the three others have idle SIMDs to
-// run on; above, the point's other work, done four times, costs more than
-// the shared scan saves. layered3 with derivatives and closure eval, us, a
-// wave's points on their own / split: 63 points 57.7 / 35.1, 4096 101.6 /
-// 46.9, 16,411 89.6 / 41.0, 32,768 81.2 / 46.1, 65,536 90.7 / 83.9, 131,072
-// 95.6 / 125.5. Of 51 generated groups with Gabor noise over 2048 unrelated
-// points 48 are faster split (216 / 137 the slowest), three alike.
-constexpr int64_t kSplitMaxPoints = 3 * 64 * 256;
 // Launches the group's own kernel over A.n > 0 points.
 int launch_group(const Group& g, GroupArgs& A, hipStream_t stream);
 

@@ -236,7 +236,7 @@ bool split_allowed(const Group& g, const GroupArgs& A)
 int launch_group(const Group& g, GroupArgs& A, hipStream_t stream)
 {
     void* args[] = { &A };
-    if (g.split && A.n <= kSplitMaxPoints && split_allowed(g, A))
+    if (g.split && A.n <= g.split_points && split_allowed(g, A))
         return check_hip(hipModuleLaunchKernel(g.split, (unsigned)((A.n + 63) / 64), 1, 1, 256, 1, 1, 0,
                                                stream, args, nullptr),
                          "hipModuleLaunchKernel(split)");

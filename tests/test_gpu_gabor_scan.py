@@ -3,7 +3,8 @@ box of cells, per lane otherwise) and of the drain of its queues, against
 the oracle's interpreter, bit for bit: boxes at and beyond the per-wave
 limits, lattice planes, partly filled waves, a noise under a branch, few and
 many impulses (the most fill a queue several times), every direction mode,
-1D to 3D, lanes with NaN or infinite coordinates. Also exp() at the ends of
+1D to 3D, lanes with NaN or infinite coordinates, in a split launch and in
+one too large to be split. Also exp() at the ends of
 its range, where the result is formed by one scaling."""
 import numpy as np
 import pytest
@@ -16,6 +17,9 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 N = 64 * 21 + 37  # the last wave is partly filled
+# copies of the points: in a launch that shares 64 points' cells among four
+# waves, and in one too large for that
+COPIES = {"split": 1, "whole": 36}
 
 
 @pytest.fixture(scope="module")
@@ -43,9 +47,10 @@ def _inputs(kind):
     return np.ascontiguousarray(P.astype(np.float32))
 
 
+@pytest.mark.parametrize("copies", COPIES.values(), ids=COPIES.keys())
 @pytest.mark.parametrize("kind", ["row", "wide", "lattice", "far"])
 @pytest.mark.parametrize("aniso,impulses", GS.SPECS)
-def test_scan_matches_interpreter(dev, kind, aniso, impulses):
+def test_scan_matches_interpreter(dev, kind, aniso, impulses, copies):
     text = GS.program(aniso, impulses)
     name = "gs_%d_%d" % (aniso, impulses)
     P = _inputs(kind)
@@ -53,18 +58,20 @@ def test_scan_matches_interpreter(dev, kind, aniso, impulses):
     ss = S.ShadingSystem()
     g = S.build_generated_group(ss, ([(name, "surface", text)], []), name, outputs=outs)
     ss.jit_group(g)
-    out = torch.full((4, N), -7.0, device=dev)
-    print("gabor scan %s %s: %d points" % (kind, name, N), flush=True)
-    ss.execute(g, N, {"P": torch.from_numpy(P).to(dev), "dPdx": (0.0,) * 3, "dPdy": (0.0,) * 3},
-               outputs=out)
+    n = N * copies
+    out = torch.full((4, n), -7.0, device=dev)
+    print("gabor scan %s %s: %d points" % (kind, name, n), flush=True)
+    ss.execute(g, n, {"P": torch.from_numpy(np.tile(P, (1, copies))).to(dev), "dPdx": (0.0,) * 3,
+                      "dPdy": (0.0,) * 3}, outputs=out)
     torch.cuda.synchronize()
     gr = O.Group([(name, "surface", text)], [])
     zero = np.zeros((3, N), np.float32)
-    got = out.cpu().numpy()
+    got = out.cpu().numpy().reshape(4, copies, N)
     for j, out_name in enumerate(outs):
         gr.outputs(out_name, "C")
         ref, _, _ = O.group_run_ex(gr, P, zero, zero, nthreads=8)
-        np.testing.assert_array_equal(got[j], ref[0], err_msg=out_name)
+        for c in range(copies):
+            np.testing.assert_array_equal(got[j, c], ref[0], err_msg="%s copy %d" % (out_name, c))
 
 
 def test_exp_range_ends(dev):
