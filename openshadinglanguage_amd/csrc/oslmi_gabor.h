@@ -250,21 +250,21 @@ OSLMI_DEV Df gabor_impulse(const GaborUniform& U, const GaborPoint& gp, V3 omega
 // own test only has to keep every impulse that passes it.
 //
 // What is left is the scan, which has two forms:
-//  * per wave: the 64 lanes shade neighbouring points, whose cells fill a
-//    small box (at most 8 x 8 x 4 and 128 cells, every lane active; the
-//    periods of a periodic noise, which wrap the cells, all alike). Each
-//    lane seeds the generator of one of the box's cells and draws its
-//    impulse count; then all lanes test every impulse of the box together.
-//    The generator runs once per wave, in the scalar unit, and nothing
-//    diverges;
-//  * per lane: each lane walks its own cells (points far apart, partly
-//    active waves).
+//  * per wave: the active lanes shade neighbouring points, whose cells fill
+//    a small box (at most 8 x 8 x 4 and 128 cells; the periods of a periodic
+//    noise, which wrap the cells, all alike). Each active lane seeds the
+//    generator of one of the box's cells and draws its impulse count; then
+//    all lanes test every impulse of the box together. The generator runs
+//    once per wave, in the scalar unit, and nothing diverges;
+//  * per lane: each lane walks its own cells (points far apart).
 // Both are bound by VALU issue. layered3 (one filtered noise in three
 // dimensions) over 1M points, the kernel where impulses are found against
-// this: 345 to 255 us; 64 generated groups over unrelated points 845 to 513
-// (32 to 2048 points each) and 1332 to 1037 us (to 262,144). A wave alone on
-// its SIMD spends 19,000 cycles on the cells' counts, 42,000 on the scan and
-// 44,000 on the queues' kernels.
+// this: 345 to 247 us; 64 generated groups over unrelated points 845 to 513
+// (32 to 2048 points each) and 1332 to 1037 us (to 262,144). A noise in three
+// dimensions under a branch that 2, 10, 30 and 90 % of 1M points take in no
+// order: 164, 187, 260 and 277 us there; 181, 210, 258 and 316 where waves
+// with an idle lane scanned per lane; 154, 143, 162 and 203 here. (At 0.4 %,
+// a lone lane in every fourth wave: 99, 114 and 105.)
 
 // Queue slots per lane: 10 slots of eight bytes for 256 work-items, 20 KB of
 // LDS: six workgroups a CU still fit, the six waves per SIMD that the
@@ -281,8 +281,7 @@ struct GaborQueued {
 // in their order, from LDS. Every wave holds the same values throughout, so
 // all of them meet at the barriers. `split` is a constant of the kernel: as
 // a value it cost the other launches 12% (registers spilled in the drain).
-// Over 16,411 points (layered3, one wave per SIMD) the evaluation falls from
-// 105,000 cycles a wave to a third, the launch from 89.6 to 41.0 us.
+// Over 16,411 points (layered3) a launch takes 42 us instead of 89.
 
 // 3039177861^k modulo 2^32: k draws of the generator at once
 constexpr uint32_t gabor_rng_pow(int k)
@@ -388,24 +387,25 @@ OSLMI_DEV GaborRng gabor_cell_rng(V3 c_i, uint32_t seed, bool periodic, V3 perio
     return GaborRng(c_i, seed);
 }
 
-// Smallest and largest value over the wave (all 64 lanes active), in every
-// lane's hands as a scalar.
+// Smallest and largest value, in 0..15, over the wave's active lanes: the
+// values' bits as lane masks, walked from the highest in scalar registers.
 #if defined(__HIP_DEVICE_COMPILE__)
-template<bool MAX> OSLMI_DEV int wave_extreme(int v)
+OSLMI_DEV void wave_range(uint32_t v, uint64_t active, int& lo, int& hi)
 {
-#define OSLMI_EXTREME_STEP(ctrl)                                                     \
-    {                                                                                \
-        const int o = __builtin_amdgcn_update_dpp(v, v, ctrl, 0xf, 0xf, false);      \
-        v           = (MAX ? o > v : o < v) ? o : v;                                 \
+    uint64_t least = active, most = active;
+    lo = hi = 0;
+#pragma unroll
+    for (int b = 3; b >= 0; --b) {
+        const uint64_t set = __ballot((v >> b) & 1u);
+        if (least & ~set)
+            least &= ~set;
+        else
+            lo |= 1 << b;
+        if (most & set) {
+            most &= set;
+            hi |= 1 << b;
+        }
     }
-    OSLMI_EXTREME_STEP(0x111)  // row_shr:1, 2, 4, 8
-    OSLMI_EXTREME_STEP(0x112)
-    OSLMI_EXTREME_STEP(0x114)
-    OSLMI_EXTREME_STEP(0x118)
-    OSLMI_EXTREME_STEP(0x142)  // row_bcast:15, 31
-    OSLMI_EXTREME_STEP(0x143)
-#undef OSLMI_EXTREME_STEP
-    return __builtin_amdgcn_readlane(v, 63);
 }
 #endif
 
@@ -432,25 +432,41 @@ struct GaborBox {
 OSLMI_DEV bool gabor_wave_box(const GaborUniform& U, V3 fl, V3 xc, GaborBox& b)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
-    if (__ballot(1) != ~0ull)
-        return false;
+    const uint64_t active = __ballot(1);
     // cells a binary32 coordinate and an int hold alike (false for NaN)
     const float lim = 1048576.0f;
     if (wave_any(!(fabsf(fl.x) < lim && fabsf(fl.y) < lim && fabsf(fl.z) < lim)))
         return false;
-    const int x = (int)fl.x, y = (int)fl.y, z = (int)fl.z;
-    b.ox = wave_extreme<false>(x) - 1;
-    b.dx = wave_extreme<true>(x) + 2 - b.ox;
-    if (b.dx > 8)
+    // the lanes' cells relative to seven below the first lane's: a larger
+    // distance does not fit a box either
+    b.ox = __builtin_amdgcn_readfirstlane((int)fl.x) - 7;
+    b.oy = __builtin_amdgcn_readfirstlane((int)fl.y) - 7;
+    b.oz = __builtin_amdgcn_readfirstlane((int)fl.z) - 7;
+    const uint32_t x = (uint32_t)((int)fl.x - b.ox), y = (uint32_t)((int)fl.y - b.oy);
+    const uint32_t z = (uint32_t)((int)fl.z - b.oz);
+    if (wave_any(x > 14u || y > 14u || z > 14u))
         return false;
-    b.oy = wave_extreme<false>(y) - 1;
-    b.dy = wave_extreme<true>(y) + 2 - b.oy;
-    b.oz = wave_extreme<false>(z) - 1;
-    b.dz = wave_extreme<true>(gabor_axis_bound(U, xc.z - 1.0f) >= U.radius2 ? z : z + 1) + 1 - b.oz;
-    return b.dy <= 8 && b.dz <= 4 && b.dx * b.dy * b.dz <= 128;
+    int lo, hi, z_hi;
+    wave_range(x, active, lo, hi);
+    b.ox += lo - 1;
+    b.dx = hi - lo + 3;
+    wave_range(y, active, lo, hi);
+    b.oy += lo - 1;
+    b.dy = hi - lo + 3;
+    wave_range(z, active, lo, hi);
+    wave_range(gabor_axis_bound(U, xc.z - 1.0f) >= U.radius2 ? z : z + 1u, active, hi, z_hi);
+    b.oz += lo - 1;
+    b.dz = z_hi - lo + 2;
+    return b.dx <= 8 && b.dy <= 8 && b.dz <= 4 && b.dx * b.dy * b.dz <= 128;
 #else
     return false;
 #endif
+}
+
+// 65536 / d + 1 for a box's size 3..8
+OSLMI_DEV int gabor_per(int d)
+{
+    return d == 3 ? 21846 : d == 4 ? 16385 : d == 5 ? 13108 : d == 6 ? 10923 : d == 7 ? 9363 : 8193;
 }
 
 // gabor_evaluate + gabor_grid: the cells around P, scaled. seed selects the
@@ -512,13 +528,16 @@ OSLMI_DEV Df gabor_grid(const GaborUniform& U, const GaborPoint& gp, const Dv& P
     int left = 0;
 #if defined(__HIP_DEVICE_COMPILE__)
     // per wave: the same of the wave's cell (wi, wj, wk), the cell-th of
-    // ncells; and the cells cell / 64 * 64 + lane, one per lane
+    // ncells; the generators of the next cells, one a lane, and the lanes
+    // whose cells are still to come
     int ncells = box.dx * box.dy * box.dz;
-    int cell = 0, cell0 = 0, wi = 0, wj = 0, wk = 0, wleft = 0, lane_count = 0;
+    int cell = 0, wi = 0, wj = 0, wk = 0, wleft = 0, lane_count = 0;
     uint32_t wcode = 0, wstate = 0, lane_state = 0;
+    uint64_t seeded = 0;
+    const int per_x = gabor_per(box.dx), per_y = gabor_per(box.dy);
     V3 wpos = at;
     if (split && by_wave) {
-        cell0       = cell = (wave * ncells) >> 2;
+        cell        = (wave * ncells) >> 2;
         ncells      = ((wave + 1) * ncells) >> 2;
         const int q = cell / box.dx;
         wi          = cell - q * box.dx;
@@ -547,9 +566,20 @@ OSLMI_DEV Df gabor_grid(const GaborUniform& U, const GaborPoint& gp, const Dv& P
 #if defined(__HIP_DEVICE_COMPILE__)
         if (by_wave) {
             if (wleft <= 0 && cell < ncells) {
-                if (((cell - cell0) & 63) == 0) {
-                    const int mine = cell + (int)__lane_id();
-                    const int q = mine / box.dx, k = q / box.dy;
+                // left out when no lane is within the radius of the cell
+                const float ex = fmaxf(fabsf(wpos.x) - 0.5f * two32, 0.0f);
+                const float ey = fmaxf(fabsf(wpos.y) - 0.5f * two32, 0.0f);
+                const float ez = fmaxf(fabsf(wpos.z) - 0.5f * two32, 0.0f);
+                const bool near
+                    = wave_any(__fmaf_rn(ez, ez, __fmaf_rn(ey, ey, ex * ex)) < near2);
+                if (near && seeded == 0) {
+                    seeded         = __ballot(1);
+                    const int mine = cell
+                                     + (int)__builtin_amdgcn_mbcnt_hi(
+                                         (uint32_t)(seeded >> 32),
+                                         __builtin_amdgcn_mbcnt_lo((uint32_t)seeded, 0));
+                    // mine / box.dx and its quotient by box.dy, both below 192
+                    const int q = (mine * per_x) >> 16, k = (q * per_y) >> 16;
                     GaborRng rng = gabor_cell_rng(
                         V3((float)(box.ox + mine - q * box.dx), (float)(box.oy + q - k * box.dy),
                            (float)(box.oz + k)),
@@ -557,15 +587,14 @@ OSLMI_DEV Df gabor_grid(const GaborUniform& U, const GaborPoint& gp, const Dv& P
                     lane_count = mine < ncells ? gabor_poisson(rng, U.poisson_g) : 0;
                     lane_state = rng.s;
                 }
-                // left out when no lane is within a cell's width of the cell
-                if (wave_any(fmaxf(fmaxf(fabsf(wpos.x), fabsf(wpos.y)), fabsf(wpos.z))
-                             < 1.50001f * two32)) {
-                    const int from = (cell - cell0) & 63;
+                if (near) {
+                    const int from = __builtin_ctzll(seeded);
                     wleft   = __builtin_amdgcn_readlane(lane_count, from);
                     wstate  = (uint32_t)__builtin_amdgcn_readlane((int)lane_state, from);
                     in_cell = wpos;
                     wcode   = gabor_cell_code(wi, wj, wk);
                 }
+                seeded &= seeded - 1;
                 // on to the next cell, x innermost
                 ++cell;
                 wpos.x -= two32;

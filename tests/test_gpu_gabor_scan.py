@@ -34,6 +34,8 @@ def _inputs(kind):
     t = np.arange(N) / 64.0
     if kind == "row":        # about four cells along x a wave
         P = np.stack([t * 3.0, 0.3 + 0.01 * t, rng.uniform(-0.4, 0.4, N)])
+    elif kind == "sparse":   # the same, one or two lanes of a wave in the branch
+        P = np.stack([t * 3.0, 0.3 + 0.01 * t, np.where(np.arange(N) % 37 == 0, 0.2, -0.2)])
     elif kind == "wide":     # about eight cells a wave: on both sides of the limit
         P = np.stack([t * 4.9, 1.7 * t, 0.2 * np.sin(t)])
     elif kind == "lattice":  # exactly on cell corners, and one step beside them
@@ -48,7 +50,7 @@ def _inputs(kind):
 
 
 @pytest.mark.parametrize("copies", COPIES.values(), ids=COPIES.keys())
-@pytest.mark.parametrize("kind", ["row", "wide", "lattice", "far"])
+@pytest.mark.parametrize("kind", ["row", "sparse", "wide", "lattice", "far"])
 @pytest.mark.parametrize("aniso,impulses", GS.SPECS)
 def test_scan_matches_interpreter(dev, kind, aniso, impulses, copies):
     text = GS.program(aniso, impulses)
