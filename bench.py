@@ -44,7 +44,7 @@ WORKLOADS = {
 # FETCH_SIZE reads half the bytes of a plain 256 MiB copy on this GPU (x2
 # scale), WRITE_SIZE reads them exactly (x1); profiles/layered3_pmc.txt. The
 # layered3 figure includes the kernel's register-spill (scratch) traffic.
-MEASURED_TRAFFIC = {"layered3": 2 * 62494.7 * 1024 + 132149.7 * 1024, "fbm_cell": None,
+MEASURED_TRAFFIC = {"layered3": 2 * 47341.0 * 1024 + 114053.0 * 1024, "fbm_cell": None,
                     # the layered closure, 2,097,152 points per launch
                     # (profiles/layered_closure_pmc.txt)
                     "closure": 2 * 107238.9 * 1024 + 262144.0 * 1024}

@@ -391,9 +391,9 @@ void parallel_for(int n, F fn)
         t.join();
 }
 
-// VGPR + AGPR count of the (single) kernel in a gfx950 code object, read
-// from its metadata note (msgpack map entries ".vgpr_count" and
-// ".agpr_count"); 0 when absent.
+// VGPR + AGPR count of the first kernel in a gfx950 code object (of a group
+// with Gabor noise, the one that is not split), read from its metadata note
+// (msgpack map entries ".vgpr_count" and ".agpr_count"); 0 when absent.
 int code_object_registers(const std::vector<char>& code)
 {
     auto field = [&](const char* key) -> int {
@@ -471,7 +471,13 @@ oslmi_batch* oslmi_batch_create(oslmi_shadingsys* s, int ngroups, oslmi_group* c
     // us eager (autotuned) at 8 / 16 / 32 groups per kernel: 32..2048 points
     // each 690 / 271 / 248, 32..262,144 points 1138 / 1107 / 1069; replayed
     // from a graph, 1155 / 736 / 408 and 1859 / 1500 / 1121. They compile in
-    // 129, 132 and 186 s; one kernel of all 64 takes 336 s, hence the limit.
+    // 129, 132 and 186 s (all kernels, one after another); one kernel of all
+    // 64 takes 336 s, hence the limit. Other batches, eager at 8 / 32, to 2048
+    // and to 262,144 points: nine generated groups 213 / 188 and 261 / 233,
+    // thirteen without Gabor noise 73 / 46 and 92 / 69, 31 generated ones and
+    // one with MaterialX closures 373 / 204 and 528 / 529; fourteen with
+    // MaterialX closures, which gain from smaller kernels, 69 / 78 and
+    // 218 / 285.
     const int per = groups_per_kernel ? groups_per_kernel : 32;
     oslmi_batch* h = new oslmi_batch;
     Batch& b       = h->b;
@@ -552,7 +558,8 @@ oslmi_batch* oslmi_batch_create(oslmi_shadingsys* s, int ngroups, oslmi_group* c
         b.any_bb = b.any_bb || p.source.find("s_bbl") != std::string::npos;
         b.parts.push_back(std::move(p));
     }
-    // compile the parts side by side (distinct hiprtc programs)
+    // compile the parts (distinct hiprtc programs; hiprtc itself compiles
+    // one at a time in a process)
     {
         const unsigned hw = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
         size_t next = 0;

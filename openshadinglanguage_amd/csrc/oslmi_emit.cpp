@@ -58,9 +58,13 @@ std::string flit(float f)
 // six / four / three / two waves): sampled 83.8 / 66.6 / 48.6 / 59.3,
 // evaluated 42.0 / 33.6 / 22.6 / 27.5, exported (21 parameters a lobe more)
 // 80.5 / 67.3 / 43.8 / 31.2. Kernels without them run best at six (layered3,
-// 1M points: 266 us; 278, 306, 301 at five, four, three). The second kernel
-// of a group with Gabor noise, launched over few points, has the three that
-// its LDS (45 KB) admits, and no spills.
+// 1M points: 266 us; 278, 306, 301 at five, four, three). MaterialX materials
+// of one lobe (sheen, dielectric, Schlick) take the same at three and at six.
+// A batch kernel that holds one MaterialX group has three for all of them: 31
+// generated groups and the layered material, 2048 to 1M points the largest,
+// take 178 to 1381 us at three and 208 to 1888 at six, whose spills the one
+// group pays for. The second kernel of a group with Gabor noise, launched
+// over few points, has the three that its LDS (45 KB) admits, and no spills.
 std::string kernel_attributes(const ShadingSys& ss, bool mx, bool exported, bool split = false)
 {
     std::string a = "__launch_bounds__(256)";
@@ -1916,8 +1920,7 @@ bool emit_batch(const ShadingSys& ss, const std::vector<Group*>& groups,
             c << "        constexpr bool split_ = false;\n";
         c << "#pragma unroll 1\n";
         c << "        for (int q_ = 0; q_ < B.ppt; ++q_) {\n";
-        c << "        int64_t i = T.begin + (int64_t)q_ * blockDim.x + "
-          << "threadIdx.x;\n";
+        c << "        int64_t i = T.begin + (int64_t)q_ * blockDim.x + threadIdx.x;\n";
         c << "        if (i < T.end) {\n";
         c << code;
         c << "        }\n        }\n";

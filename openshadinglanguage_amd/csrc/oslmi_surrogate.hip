@@ -599,8 +599,9 @@ __device__ __forceinline__ void run_tiles(const InferLds& L, int wv, int head, i
 // compaction, query order kept). Whenever 32 are queued, the network runs
 // on two 16-query tiles; the rest is flushed after the last chunk. The next
 // chunk's inputs are loaded before the network runs on the current queue.
-// What bounds it is the SiLU: of the about 4200 issue cycles that 32 queries
-// take, 256 exp2 and rcp take 2900. Measured over 8M queries, 4.19M of them
+// What bounds it is the SiLU: of the 812 VALU instructions that 32 queries
+// take 256 are exp2 and rcp, which issue at a quarter of the rate, and the
+// VALU is busy 76 % of the time. Measured over 8M queries, 4.19M of them
 // for the network (with the exact fallback): 350 us; 412 with the weights in
 // the accumulation registers, the ring in fp32 and two waves per SIMD; 397
 // with five waves (ten to a workgroup: two SIMDs carry more); 353 with

@@ -14,6 +14,7 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 MOST = 3 * 64 * 256  # points of the largest split launch
+LIMIT = "split launches: up to %d points" % MOST
 SIZES = [1, 63, 64, 65, 64 * 21 + 37, MOST]
 
 
@@ -46,6 +47,7 @@ def test_split_matches_whole(dev, aniso, impulses):
     ss = S.ShadingSystem()
     g = S.build_generated_group(ss, ([(name, "surface", GS.program(aniso, impulses))], []), name,
                                 outputs=GS.OUTPUTS)
+    assert LIMIT in ss.emit(g)
     ss.jit_group(g)
     P = _points(dev)
     zero = {"dPdx": (0.0,) * 3, "dPdy": (0.0,) * 3}
@@ -72,6 +74,7 @@ def test_split_matches_whole(dev, aniso, impulses):
 def test_split_layered3(dev, n):
     """Filtered Gabor noise with derivatives, closure evaluated."""
     ss, g = S.build_layered3()
+    assert LIMIT in ss.emit(g)
     ss.jit_group(g)
     d = torch.nn.functional.normalize(torch.randn((3, MOST + 1), device=dev,
                                                   generator=torch.Generator(dev).manual_seed(7)), dim=0)
